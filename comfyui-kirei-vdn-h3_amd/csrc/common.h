@@ -137,6 +137,13 @@ __device__ __forceinline__ void wait_vm_lds() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
 }
 
+// s_waitcnt with vmcnt <= N only: LDS reads stay in flight.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
 // Workgroup barrier without the fence of __syncthreads (which would also wait for every
 // in-flight tile load); the empty asm statements keep the compiler from moving memory
 // accesses across it. The waits the step needs are issued explicitly before it.

@@ -238,3 +238,47 @@ def test_full_shape_int8_out_projection_sampled(device):
     assert torch.equal(acc[rows.to(device)].cpu(), want_acc)
     want = qo.int8_linear(xq[rows.to(device)].cpu(), xs[rows.to(device)].cpu(), wq.cpu(), ws.cpu().reshape(1, -1))
     assert_bf16_close(out[rows.to(device)], want, steps=1)
+
+
+# one size per tile height the launcher can pick (32 mi rows: the fewest rounds over 256 CUs), each with a ragged
+# last tile row, N a multiple of 8, of 4 and odd (the three store widths), and 1 to 5 stages of 128 K bytes
+@pytest.mark.parametrize("stages", [1, 2, 3, 5])
+@pytest.mark.parametrize("m,n", [(1, 8), (31, 20), (65, 257), (513, 15100), (1801, 5113), (2303, 5116), (2561, 5120),
+                                 (2881, 4900), (4100, 5128)])
+def test_tile_heights_widths_and_stages(device, m, n, stages):
+    from vdn_h3_amd import linear
+
+    print(f"case tiles {m}x{n}, {stages} stages", flush=True)
+    # int8: exact integers; the bf16 output rounds acc * a_scale * b_scale once
+    k = 128 * stages
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n + stages)
+    aq = torch.randint(-127, 128, (m, k), generator=g, device=device, dtype=torch.int8)
+    bq = torch.randint(-127, 128, (n, k), generator=g, device=device, dtype=torch.int8)
+    a_s = torch.rand(m, 1, generator=g, device=device) * 1e-2
+    b_s = torch.rand(1, n, generator=g, device=device) * 1e-2
+    acc = (aq.float() @ bq.float().t())  # at most 640 products below 2^14: exact in fp32
+    assert torch.equal(linear.int8_accumulators(aq, bq), acc.to(torch.int32))
+    assert torch.equal(linear.gemm_w8a8(aq, a_s, bq, b_s), (acc * a_s * b_s).to(torch.bfloat16))
+    assert torch.equal(linear.gemm_w8a8(aq, a_s, bq, b_s, out_dtype=torch.float32), acc * a_s * b_s)
+    # bf16: fp32 sums of K products; fp8: the instruction keeps about 15 bits below the largest products it sums
+    # (measured: at most 2^-15 of sum |a b| off the exact sum, in its 32x32 and 16x16 shapes alike). Then one
+    # rounding (2^-9 relative; 2^-8 leaves room for a tie).
+    for kind in ("fp8", "bf16"):
+        k = (128 if kind == "fp8" else 64) * stages
+        a = torch.randn(m, k, generator=g, device=device).to(torch.bfloat16)
+        b = (torch.randn(n, k, generator=g, device=device) * 0.1).to(torch.bfloat16)
+        base = torch.randn(m, n, generator=g, device=device).to(torch.bfloat16)
+        out = base.clone()
+        if kind == "fp8":
+            a, b = a.to(torch.float8_e4m3fn), b.to(torch.float8_e4m3fn)
+            one = torch.ones(1, 1, device=device)
+            got = linear.gemm_w8a8(a, one, b, one)
+            linear.gemm_w8a8(a, one, b, one, out=out, accumulate=True)
+        else:
+            got = linear.linear(a, b)
+            linear.linear(a, b, out=out, accumulate=True)
+        ad, bd = a.double(), b.double()
+        want = ad @ bd.t()
+        bound = (2.0 ** -14 if kind == "fp8" else k * 2.0 ** -24) * (ad.abs() @ bd.abs().t())
+        assert bool(((got.double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()), kind
+        assert torch.equal(out, (base.float() + got.float()).to(torch.bfloat16)), kind
