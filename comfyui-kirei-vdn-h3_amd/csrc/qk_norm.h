@@ -34,16 +34,18 @@ __device__ __forceinline__ float group_tree_sum(float p) {
   return p;
 }
 
-// The same tree over NC = 2 * M chunk partials when chunk 2s + g sits in element s of lane half g
-// (g = lane / 32) of a wavefront: first the pairs (2s, 2s + 1) across the half-waves through
-// v_permlane32_swap, then the local pairwise tree over s.
+// The same tree over NC = 4 * M chunk partials when chunk 4s + g sits in element s of the 16-lane group g
+// (g = lane / 16) of a wavefront: first the pairs (4s, 4s + 1), (4s + 2, 4s + 3) through
+// v_permlane16_swap, then those across the half-waves (v_permlane32_swap), then the local tree over s.
 template <int M>
-__device__ __forceinline__ float halves_tree_sum(const float (&p)[M]) {
+__device__ __forceinline__ float quarters_tree_sum(const float (&p)[M]) {
   float q[M];
 #pragma unroll
   for (int s = 0; s < M; ++s) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[s]), __float_as_uint(p[s]), false, false);
-    q[s] = __uint_as_float(r[0]) + __uint_as_float(r[1]);  // low half's chunk 2s plus high half's 2s + 1
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(p[s]), __float_as_uint(p[s]), false, false);
+    const uint32_t x = __float_as_uint(__uint_as_float(a[0]) + __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    q[s] = __uint_as_float(b[0]) + __uint_as_float(b[1]);
   }
 #pragma unroll
   for (int w = 1; w < M; w <<= 1)

@@ -6,11 +6,14 @@
 //
 // Work decomposition
 //   one workgroup = 8 wavefronts = 256 query rows of one head x the key tiles of its run;
-//   each wavefront owns 32 query rows and keeps its Q fragment in registers.
-//   Scores are computed transposed, S^T = K Q^T, with v_mfma_f32_32x32x16_bf16: every lane
-//   then owns one query column (lane % 32) and 3 x 16 of the 96 keys of a tile, so the row
-//   max is one cross-lane exchange (lane ^ 32) and the probabilities P^T feed the next
-//   MFMA (O^T += V^T P^T) straight from registers, without an LDS round trip.
+//   each wavefront owns 32 query rows and keeps its Q fragments in registers.
+//   Scores are computed transposed, S^T = K Q^T, with v_mfma_f32_16x16x32_bf16: every lane
+//   then owns one query of each 16-query block (lane % 16) and 24 of the 96 keys of a tile, so the row
+//   maxima take three lane swaps and the probabilities P^T feed the next MFMA (O^T += V^T P^T)
+//   straight from registers, without an LDS round trip. The 16x16 shape does the same work at 13% less
+//   power than 32x32x16 (register-only rates 2003 against 1740 TFLOP/s on random operands), and this kernel
+//   is power-bound: with the row sums below, 15.55 -> 15.02 ms at 40,688 x 40 x 128 and 2510 -> 2368 us at
+//   16,007 x 56 x 128 (72 frames of 209 tokens), alternated on one machine.
 //   V^T is read from a copy made by a pre-pass (one extra 2*S*H*D-byte sweep): per head, one
 //   contiguous image per 96-key tile, its 16-byte chunks already in the order and XOR swizzle of
 //   the kernel's LDS tile, with keys interleaved in 16-key groups so that each lane's 8 MFMA
@@ -35,11 +38,14 @@ constexpr int kBM = 256;  // query rows per workgroup (8 wavefronts x 32)
 constexpr int kBN = 96;   // keys per tile: 48 MFMAs per wavefront and phase at D = 128
 constexpr int kThreads = 512;
 constexpr int kRing = 3;  // LDS slots per K and V^T ring (144 KB at D = 128): loads run kRing - 1 tiles ahead
+// fragments a wavefront's LDS reads run ahead of its MFMAs: 8 / 6 / 5 / 4 measured 15.45 / 15.31 / 15.17 / 15.39 ms
+// at the full shape, and with the row sums as MFMAs 6 / 5 / 4 15.04 / 15.09 / 15.02
+constexpr int kAhead = 4;
 constexpr float kLazy = 8.0f;  // log2 of the largest probability a stale running max allows
 
-// LDS position p (0..15) inside a 16-key group holds key offset kperm(p): the order in
-// which the S^T accumulator of lane group g = p / 8 enumerates its 8 keys of a k-step.
-__host__ __device__ constexpr int kperm(int p) { return 8 * ((p & 7) >> 2) + 4 * (p >> 3) + (p & 3); }
+// LDS position p (0..31) inside a 32-key group holds key offset kperm(p): the order in which lane
+// group g = p / 8 holds its 8 keys of a k-step in two 16x16 blocks of S^T.
+__host__ __device__ constexpr int kperm(int p) { return 16 * ((p & 7) >> 2) + 4 * (p >> 3) + (p & 3); }
 
 // ---------------------------------------------------------------------------------
 // LDS slots of the staged tiles. Each tile row is split into 16-byte chunks; chunk c of row r
@@ -66,10 +72,10 @@ __host__ __device__ constexpr int pad_rows(int seq) { return (seq + 191) / 192 *
 // order: position P < 8 D is (d = P / 8, slot P % 8) of the 64-key part, holding chunk
 // v_slot(d, slot) of keys [ks, ks + 64) of V^T row d; position 8 D + 4 d + slot of the 32-key part
 // holds chunk vb_slot(d, slot) of keys [ks + 64, ks + 96). Inside a chunk the 8 keys follow kperm
-// within their 16-key group; keys past seq are zero. A tile load is then a contiguous copy.
+// within their 32-key group; keys past seq are zero. A tile load is then a contiguous copy.
 // write_vt_image: the image chunks of the 64 keys [k0, k0 + 64) (k0 a multiple of 64) from their V rows
 // staged in LDS (row r at rows + r * P), into the head's images at vt_head. A 64-key block holds whole
-// 16-key groups, so every chunk it writes is complete; it covers one or two tiles.
+// 32-key groups, so every chunk it writes is complete; it covers one or two tiles.
 template <int D, int P>
 __device__ __forceinline__ void write_vt_image(const uint16_t *rows, int k0, uint16_t *__restrict__ vt_head,
                                                int tid) {
@@ -81,7 +87,7 @@ __device__ __forceinline__ void write_vt_image(const uint16_t *rows, int k0, uin
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int p = 8 * pc + j;
-      e[j] = rows[((p & ~15) + kperm(p & 15)) * P + d];
+      e[j] = rows[((p & ~31) + kperm(p & 31)) * P + d];
     }
     uint4 o;
     o.x = uint32_t(e[0]) | (uint32_t(e[1]) << 16);
@@ -239,80 +245,85 @@ __global__ __launch_bounds__(kThreads) void qkv_prepass_kernel(
 
 
 
-// The value of lane (l + 32) mod 64, via v_permlane32_swap (gfx950).
-__device__ __forceinline__ float other_half(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const uint32_t lane = __lane_id();
-  return __uint_as_float(lane < 32 ? r[1] : r[0]);
+// Reductions over the four 16-lane groups of a wavefront through v_permlane32_swap / v_permlane16_swap (gfx950).
+// lanes < 32: max of a over lane groups (g, g + 2); lanes >= 32: the same of b
+__device__ __forceinline__ float max_pair32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// a over the four lane groups, b over the four lane groups, each in every lane
+__device__ __forceinline__ void group_max(float &a, float &b) {
+  const uint32_t x = __float_as_uint(max_pair32(a, b));
+  const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const uint32_t y = __float_as_uint(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+  const auto q = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  a = __uint_as_float(q[0]);
+  b = __uint_as_float(q[1]);
 }
 
-// The Q^T fragments of a wavefront: lane (l32, g) holds channels 16 s + 8 g + j (j < 8) of its
-// query row qrc, chunk 2 s + g. QNORM: q is normalised as it is loaded (the block's q_norm with
-// q_weight / q_eps, the arithmetic of qk_norm.h); otherwise q is used as given.
+constexpr int kNQ = 2;  // 16-query blocks per wavefront
+
+// The Q^T fragments of a wavefront: lane (l16, g) holds channels 32 s + 8 g + j (j < 8) of query rows
+// q0 + 16 n + l16, chunk 4 s + g (rows at or past q1 read row q1 - 1). QNORM: q is normalised as it is
+// loaded (the block's q_norm with q_weight / q_eps, the arithmetic of qk_norm.h); otherwise q is used as given.
 template <int D, bool QNORM>
-__device__ __forceinline__ void load_q_frags(const uint16_t *__restrict__ q, int64_t q_row, int64_t q_head, int qrc,
-                                             int head, int g, const uint16_t *__restrict__ q_weight, float q_eps,
-                                             bf16x8_t (&qf)[D / 16]) {
-  constexpr int NS = D / 16;
-  const uint16_t *qp = q + (int64_t)qrc * q_row + (int64_t)head * q_head + 8 * g;
-  if constexpr (!QNORM) {
+__device__ __forceinline__ void load_q_frags(const uint16_t *__restrict__ q, int64_t q_row, int64_t q_head, int q0,
+                                             int q1, int head, int l16, int g, const uint16_t *__restrict__ q_weight,
+                                             float q_eps, bf16x8_t (&qf)[kNQ][D / 32]) {
+  constexpr int NS = D / 32;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) qf[s] = as_bf16x8(ld16(qp + 16 * s));
-  } else {
-    float y[NS][8], p[NS];
+  for (int n = 0; n < kNQ; ++n) {
+    const uint16_t *qp = q + (int64_t)min(q0 + 16 * n + l16, q1 - 1) * q_row + (int64_t)head * q_head + 8 * g;
+    if constexpr (!QNORM) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const u32x4_t raw = ld16(qp + 16 * s);
+      for (int s = 0; s < NS; ++s) qf[n][s] = as_bf16x8(ld16(qp + 32 * s));
+    } else {
+      float y[NS][8], p[NS];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        y[s][j] = __uint_as_float((j & 1) ? (raw[j >> 1] & 0xffff0000u) : (raw[j >> 1] << 16));
-      p[s] = chunk_sumsq(y[s]);
+      for (int s = 0; s < NS; ++s) {
+        const u32x4_t raw = ld16(qp + 32 * s);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          y[s][j] = __uint_as_float((j & 1) ? (raw[j >> 1] & 0xffff0000u) : (raw[j >> 1] << 16));
+        p[s] = chunk_sumsq(y[s]);
+      }
+      const float rr = rms_factor(quarters_tree_sum<NS>(p), D, q_eps);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const u32x4_t w = ld16(q_weight + 32 * s + 8 * g);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          y[s][j] = y[s][j] * rr * __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
+        qf[n][s] = as_bf16x8(u32x4_t{pack_bf2(y[s][0], y[s][1]), pack_bf2(y[s][2], y[s][3]),
+                                     pack_bf2(y[s][4], y[s][5]), pack_bf2(y[s][6], y[s][7])});
+      }
     }
-    const float rr = rms_factor(halves_tree_sum<NS>(p), D, q_eps);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const u32x4_t w = ld16(q_weight + 16 * s + 8 * g);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        y[s][j] = y[s][j] * rr * __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
-    }
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      qf[s] = as_bf16x8(u32x4_t{pack_bf2(y[s][0], y[s][1]), pack_bf2(y[s][2], y[s][3]), pack_bf2(y[s][4], y[s][5]),
-                                pack_bf2(y[s][6], y[s][7])});
   }
 }
 
-// The output rows of a wavefront: O = O^T / l (l summed over the two half-waves), rounded to bf16,
-// times the row's gate when one is given (the gate fused into the attention epilogue).
+// The output rows of a wavefront: O = O^T / l, rounded to bf16, times the row's gate when one is given
+// (the gate fused into the attention epilogue). Every element of l[n] holds the row sum of the lane's query.
 template <int D>
-__device__ __forceinline__ void store_rows(const f32x16_t (&oacc)[D / 32], float l_run, int qr, int q1,
-                                           const uint16_t *__restrict__ gate, int64_t g_row, int head,
-                                           uint16_t *__restrict__ out, int64_t o_row, int64_t o_head, int g) {
-  constexpr int NO = D / 32;
-  l_run += other_half(l_run);
-  const float inv = 1.f / l_run;
-  if (qr < q1) {
-    float gv = 1.f;
-    if (gate) gv = bf2f(gate[(int64_t)qr * g_row + head]);
-    uint16_t *op = out + (int64_t)qr * o_row + (int64_t)head * o_head;
+__device__ __forceinline__ void store_rows(const f32x4_t (&oacc)[D / 16][kNQ], const f32x4_t (&l)[kNQ], int q0,
+                                           int q1, const uint16_t *__restrict__ gate, int64_t g_row, int head,
+                                           uint16_t *__restrict__ out, int64_t o_row, int64_t o_head, int l16, int g) {
 #pragma unroll
-    for (int m = 0; m < NO; ++m)
+  for (int n = 0; n < kNQ; ++n) {
+    const float inv = 1.f / l[n][0];
+    const int qr = q0 + 16 * n + l16;
+    if (qr >= q1) continue;
+    const float gv = gate ? bf2f(gate[(int64_t)qr * g_row + head]) : 1.f;
+    uint16_t *op = out + (int64_t)qr * o_row + (int64_t)head * o_head + 4 * g;
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        float v0 = round_bf(oacc[m][4 * i4 + 0] * inv), v1 = round_bf(oacc[m][4 * i4 + 1] * inv);
-        float v2 = round_bf(oacc[m][4 * i4 + 2] * inv), v3 = round_bf(oacc[m][4 * i4 + 3] * inv);
-        if (gate) {
-          v0 *= gv;
-          v1 *= gv;
-          v2 *= gv;
-          v3 *= gv;
-        }
-        uint2 w;
-        w.x = pack_bf2(v0, v1);
-        w.y = pack_bf2(v2, v3);
-        *reinterpret_cast<uint2 *>(op + 32 * m + 8 * i4 + 4 * g) = w;
+    for (int m = 0; m < D / 16; ++m) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = round_bf(oacc[m][n][r] * inv);
+        if (gate) v[r] *= gv;
       }
+      *reinterpret_cast<uint2 *>(op + 16 * m) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+    }
   }
 }
 
@@ -321,15 +332,17 @@ __device__ __forceinline__ void store_rows(const f32x16_t (&oacc)[D / 32], float
 // Waves 0-3 (group A) and 4-7 (group B) each own 32 query rows; wave w and w + 4 share a SIMD.
 // The item runs in barrier-separated phases p = 0 .. 2T+1; in each phase one group works on the
 // matrix cores and the other on the VALU, so the two waves of every SIMD alternate:
-//   MFMA phase of tile t :  O^T += V(t-1)^T P(t-1)^T   and   S(t)^T = K(t) Q^T      (48 MFMAs)
-//   VALU phase of tile t :  P(t) = exp2(scale S(t) - m), row max / sum, O rescale   (softmax)
+//   MFMA phase of tile t :  O^T += V(t-1)^T P(t-1)^T, l += 1^T P(t-1)^T, S(t)^T = K(t) Q^T  (102 MFMAs)
+//   VALU phase of tile t :  P(t) = exp2(scale S(t) - m), row max, O and l rescale   (softmax)
 // Group A runs tile t's MFMA phase in phase 2t and its VALU phase in 2t+1; group B one phase
 // later. K(t) and V(t-1) are read in phases 2t and 2t+1 only; tiles are loaded direct to LDS
 // into three-slot rings, two tiles ahead: K tiles by group A and V^T tiles by group B, each at
 // the start of the issuing group's VALU phase, so the MFMA stream carries no memory instruction
 // and a tile that misses L2 has two tiles' time to land. A tile is 96 keys: every phase switch
-// (a barrier, the first fragment reads of the MFMA phase) is shared by 48 MFMAs per wavefront, a
-// third fewer switches than with 64-key tiles for the same work.
+// (a barrier, the first fragment reads of the MFMA phase) is shared by 96 16x16 MFMAs per wavefront, a
+// third fewer switches than with 64-key tiles for the same work. The VALU phase is the longer one, so the row
+// sums of P are six more MFMAs against a fragment of ones instead of 24 dot products in it (and come out
+// summed over the lane groups): 15.30 -> 15.06 ms at 40,688 x 40 x 128, 2406 -> 2370 us at 16,007 x 56 x 128.
 // QNORM: q is normalised as it is loaded (the block's q_norm with q_weight / q_eps, the arithmetic
 // of qk_norm.h); otherwise q is used as given.
 template <int D, bool QNORM>
@@ -340,10 +353,10 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
     const int4 *__restrict__ items, int n_items, const int2 *__restrict__ tiles, int per_xcd, int total,
     const uint16_t *__restrict__ q_weight, float q_eps) {
   constexpr int KC = D / 8;    // 16-byte chunks per K row
-  constexpr int NS = D / 16;   // k-steps of the QK^T contraction
-  constexpr int NO = D / 32;   // 32-row blocks of O^T
-  constexpr int NKB = kBN / 32;  // 32-key blocks of S^T
-  constexpr int NT = kBN / 16;   // k-steps of the PV contraction
+  constexpr int NS = D / 32;   // k-steps of the QK^T contraction
+  constexpr int NO = D / 16;   // 16-row blocks of O^T
+  constexpr int NKB = kBN / 16;  // 16-key blocks of S^T
+  constexpr int NT = kBN / 32;   // k-steps of the PV contraction
   constexpr int KT = kBN * D, VT = D * kBN;  // elements per tile
   // a V^T tile in LDS: keys 0..63 as [D][8 chunks] (v_slot), then keys 64..95 as [D][4 chunks] (vb_slot)
   constexpr int VA = D * 64;
@@ -359,17 +372,15 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   const int q0 = item.x, q1 = item.y, toff = item.z, T = item.w;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int l32 = lane & 31, g = lane >> 5;
+  const int l16 = lane & 15, g = lane >> 4;
   const int group = wave >> 2;
-  const int qr = q0 + wave * 32 + l32;
-  const int qrc = min(qr, q1 - 1);
   // a wavefront whose 32 rows all lie past the item's end (the short last item of a run) skips
   // its fragment reads, MFMAs and softmax; it still issues its share of the tile loads and
   // joins every barrier
   const bool rows_live = q0 + wave * 32 < q1;
 
-  bf16x8_t qf[NS];
-  load_q_frags<D, QNORM>(q, q_row, q_head, qrc, head, g, q_weight, q_eps, qf);
+  bf16x8_t qf[kNQ][NS];
+  load_q_frags<D, QNORM>(q, q_row, q_head, q0 + wave * 32, q1, head, l16, g, q_weight, q_eps, qf);
 
   const uint16_t *kbase = k + (int64_t)head * k_head;
   const uint16_t *vbase = vt + (int64_t)head * D * s_pad;
@@ -414,21 +425,28 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   };
 
   // Fragment offsets inside a tile (elements). The swizzles depend on the row only through
-  // l32 (r = 32 kb + l32, d = 32 m + l32), so the 32-row blocks differ by constant offsets.
+  // l16 (r = 16 kb + l16, d = 16 m + l16), so the 16-row blocks differ by constant offsets.
   int kfo[NS], vfo[NT];
 #pragma unroll
-  for (int st = 0; st < NS; ++st) kfo[st] = (l32 * KC + k_slot<D>(l32, 2 * st + g)) * 8;
+  for (int st = 0; st < NS; ++st) kfo[st] = (l16 * KC + k_slot<D>(l16, 4 * st + g)) * 8;
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt)
-    vfo[tt] = tt < 4 ? (l32 * 8 + v_slot(l32, 2 * tt + g)) * 8 : VA + (l32 * 4 + vb_slot(l32, 2 * (tt - 4) + g)) * 8;
+    vfo[tt] = tt < 2 ? (l16 * 8 + v_slot(l16, 4 * tt + g)) * 8 : VA + (l16 * 4 + vb_slot(l16, g)) * 8;
 
-  f32x16_t oacc[NO], sacc[NKB];
+  f32x4_t oacc[NO][kNQ], sacc[NKB][kNQ];
+  u32x4_t pb[NT][kNQ];  // P^T fragments: bf16 pairs
+  f32x4_t l_run[kNQ];    // row sums of P: every element of a lane's vector is its query's sum
+  const u32x4_t ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // eight bf16 1.0
+  float m_run[kNQ];
 #pragma unroll
-  for (int m = 0; m < NO; ++m) oacc[m] = f32x16_t{};
-  bf16x8_t pb[NT];
+  for (int n = 0; n < kNQ; ++n) {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) pb[j] = bf16x8_t{};
-  float m_run = -INFINITY, l_run = 0.f;
+    for (int m = 0; m < NO; ++m) oacc[m][n] = f32x4_t{};
+#pragma unroll
+    for (int j = 0; j < NT; ++j) pb[j][n] = u32x4_t{};
+    m_run[n] = -INFINITY;
+    l_run[n] = f32x4_t{};
+  }
 
   // Rings: K(tau) and V(tau) live in slot tau % kRing. K(t) and V(t-1) are read in phases 2t
   // (group A) and 2t+1 (group B). Tile loads are issued by the group in its VALU phase, so the
@@ -466,40 +484,47 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
         // descriptors of this group's next VALU phase (tile t_mfma)
         dma_ks = tiles[toff + min(t_mfma + kRing - 1, T - 1)].x;
       } else {
-      // MFMA phase of tile t: O^T += V(t-1)^T P(t-1)^T, S(t)^T = K(t) Q^T (24 + 24 MFMAs at D = 128).
+      // MFMA phase of tile t: O^T += V(t-1)^T P(t-1)^T, S(t)^T = K(t) Q^T (48 + 48 MFMAs at D = 128) and
+      // l += 1^T P(t-1)^T (6).
       // t = 0 has no PV and t = T no QK: those phases run on a zero tile / discard the scores,
-      // so the phase is one branch-free block. Fragment reads run eight MFMAs ahead.
+      // so the phase is one branch-free block. Fragment reads run kAhead fragments ahead.
       const int t = t_mfma;
       const uint16_t *vtile = Vs[(t + kRing - 1) % kRing];
       const uint16_t *ktile = Ks[t % kRing];
-      // MFMA i < NP: PV block m = i % NO, k-step tt = i / NO; i >= NP: QK block kb = (i - NP) % NKB,
-      // k-step st = (i - NP) / NKB. Consecutive MFMAs update different accumulators, so none waits
-      // for the result of the one before it.
-      constexpr int NP = NO * NT, NM = NP + NKB * NS;
+      // fragment i < NP: V^T block m = i % NO, k-step tt = i / NO; i >= NP: K block kb = (i - NP) % NKB,
+      // k-step st = (i - NP) / NKB. Each feeds kNQ MFMAs (one per query block), the query blocks in
+      // alternating order, so successive MFMAs share an operand (less toggling, less power) and none
+      // waits for the result of the one before it.
+      constexpr int NP = NO * NT, NF = NP + NKB * NS;
       auto frag = [&](int i) __device__ {
         if (i < NP) {
           const int m = i % NO, tt = i / NO;
-          return ld16(vtile + (tt < 4 ? m * 32 * 64 : m * 32 * 32) + vfo[tt]);
+          return ld16(vtile + (tt < 2 ? m * 16 * 64 : m * 16 * 32) + vfo[tt]);
         }
-        return ld16(ktile + ((i - NP) % NKB) * 32 * D + kfo[(i - NP) / NKB]);
+        return ld16(ktile + ((i - NP) % NKB) * 16 * D + kfo[(i - NP) / NKB]);
       };
       // the MFMA wave of each SIMD issues ahead of the VALU wave sharing it
       __builtin_amdgcn_s_setprio(1);
-      u32x4_t fr[8];
+      u32x4_t fr[kAhead];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) fr[i] = frag(i);
+      for (int i = 0; i < kAhead; ++i) fr[i] = frag(i);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < NM; ++i) {
-        const u32x4_t a = fr[i & 7];
-        if (i < NP) {
-          oacc[i % NO] = mfma_bf16_32x32x16(as_bf16x8(a), pb[i / NO], oacc[i % NO]);
-        } else {
-          const int kb = (i - NP) % NKB, st = (i - NP) / NKB;
-          if (st == 0) sacc[kb] = f32x16_t{};
-          sacc[kb] = mfma_bf16_32x32x16(as_bf16x8(a), qf[st], sacc[kb]);
+      for (int i = 0; i < NF; ++i) {
+        const u32x4_t a = fr[i % kAhead];
+#pragma unroll
+        for (int x = 0; x < kNQ; ++x) {
+          const int n = (i & 1) ? kNQ - 1 - x : x;
+          if (i < NP) {
+            oacc[i % NO][n] = mfma_bf16_16x16x32(as_bf16x8(a), as_bf16x8(pb[i / NO][n]), oacc[i % NO][n]);
+            if (i % NO == NO - 1) l_run[n] = mfma_bf16_16x16x32(as_bf16x8(ones), as_bf16x8(pb[i / NO][n]), l_run[n]);
+          } else {
+            const int kb = (i - NP) % NKB, st = (i - NP) / NKB;
+            if (st == 0) sacc[kb][n] = f32x4_t{};
+            sacc[kb][n] = mfma_bf16_16x16x32(as_bf16x8(a), qf[n][st], sacc[kb][n]);
+          }
         }
-        if (i + 8 < NM) fr[i & 7] = frag(i + 8);
+        if (i + kAhead < NF) fr[i % kAhead] = frag(i + kAhead);
         __builtin_amdgcn_sched_barrier(0);
       }
       __builtin_amdgcn_s_setprio(0);
@@ -509,9 +534,10 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
       }
     } else {
       // VALU phase of tile t: first this group's tile loads (two tiles ahead), then the softmax
-      // in base 2, one query per lane. The running max m_run moves only when this tile's max
-      // exceeds it by more than 2^kLazy: probabilities stay below 2^kLazy (exact softmax either
-      // way, a common shift cancels in O / l) and most tiles skip the rescale.
+      // in base 2; a lane holds 24 of the 96 scores of each of its two queries. The running max m_run
+      // moves only when this tile's max exceeds it by more than 2^kLazy: probabilities stay below
+      // 2^kLazy (exact softmax either way, a common shift cancels in O / l) and most tiles skip the
+      // rescale.
       tile_dma(dma_ks, (t_valu + kRing - 1) % kRing);
       const bool work = rows_live && p >= 1 + group && t_valu < T;
       if (work) {
@@ -520,51 +546,58 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
 #pragma unroll
           for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int ko = 32 * kb + 8 * (i >> 2) + 4 * g + (i & 3);
-              if (ko < lo || ko >= hi) sacc[kb][i] = -INFINITY;
+            for (int i = 0; i < 4; ++i) {
+              const int ko = 16 * kb + 4 * g + i;
+              if (ko < lo || ko >= hi) {
+#pragma unroll
+                for (int n = 0; n < kNQ; ++n) sacc[kb][n][i] = -INFINITY;
+              }
             }
         }
-        // tile row max over the lane's 48 scores as a tree of three-input maxima (16 + 5 + 2
-        // v_max3), then the other half-wave's value through v_permlane32_swap (no LDS round trip)
-        static_assert(NKB == 3, "the max tree is written for 48 scores per lane");
-        float m1[16];
+        // tile row max over the lane's 24 scores of a query as a tree of three-input maxima (8 + 3
+        // v_max3), then over the four lane groups for both queries in three lane swaps
+        static_assert(NKB == 6 && kNQ == 2, "the max tree is written for 2 x 24 scores per lane");
+        float mt[kNQ];
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          m1[i] = fmaxf(fmaxf(sacc[0][i], sacc[1][i]), sacc[2][i]);
-        float m2[6];
+        for (int n = 0; n < kNQ; ++n) {
+          float m1[8];
 #pragma unroll
-        for (int i = 0; i < 5; ++i) m2[i] = fmaxf(fmaxf(m1[3 * i], m1[3 * i + 1]), m1[3 * i + 2]);
-        m2[5] = m1[15];
-        const float mx = fmaxf(fmaxf(fmaxf(m2[0], m2[1]), m2[2]), fmaxf(fmaxf(m2[3], m2[4]), m2[5]));
-        const float mt = fmaxf(mx, other_half(mx)) * scale_log2;
-        const bool grow = mt > m_run + kLazy;
-        if (__any(grow)) {
-          const float m_new = grow ? mt : m_run;
-          const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
-          m_run = m_new;
-          l_run *= corr;
-#pragma unroll
-          for (int m = 0; m < NO; ++m) oacc[m] *= corr;
+          for (int i = 0; i < 4; ++i) {
+            m1[i] = fmaxf(fmaxf(sacc[0][n][i], sacc[1][n][i]), sacc[2][n][i]);
+            m1[4 + i] = fmaxf(fmaxf(sacc[3][n][i], sacc[4][n][i]), sacc[5][n][i]);
+          }
+          const float a = fmaxf(fmaxf(m1[0], m1[1]), m1[2]), b = fmaxf(fmaxf(m1[3], m1[4]), m1[5]);
+          mt[n] = fmaxf(fmaxf(a, b), fmaxf(m1[6], m1[7]));
         }
-        // P in bf16 pairs; the row sum adds the bf16 values the PV product uses, two per
-        // v_dot2c_f32_bf16 against (1, 1), in four independent chains
-        typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-        const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
-        float rs[4] = {0.f, 0.f, 0.f, 0.f};
+        group_max(mt[0], mt[1]);
+        bool grow = false;
+#pragma unroll
+        for (int n = 0; n < kNQ; ++n) {
+          mt[n] *= scale_log2;
+          grow = grow || mt[n] > m_run[n] + kLazy;
+        }
+        if (__any(grow)) {
+#pragma unroll
+          for (int n = 0; n < kNQ; ++n) {
+            const float m_new = mt[n] > m_run[n] + kLazy ? mt[n] : m_run[n];
+            const float corr = __builtin_amdgcn_exp2f(m_run[n] - m_new);
+            m_run[n] = m_new;
+            l_run[n] *= corr;
+#pragma unroll
+            for (int m = 0; m < NO; ++m) oacc[m][n] *= corr;
+          }
+        }
+        // P in bf16 pairs (the values the PV product and the row sums use)
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-          for (int i = 0; i < 16; i += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[kb][i], scale_log2, -m_run));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[kb][i + 1], scale_log2, -m_run));
-            const uint32_t pk = pack_bf2(p0, p1);
-            pb[2 * kb + (i >> 3)][i & 7] = __builtin_bit_cast(__bf16, (uint16_t)(pk & 0xffffu));
-            pb[2 * kb + (i >> 3)][(i & 7) + 1] = __builtin_bit_cast(__bf16, (uint16_t)(pk >> 16));
-            rs[(i >> 1) & 3] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk), ones,
-                                                               rs[(i >> 1) & 3], false);
-          }
-        l_run += (rs[0] + rs[1]) + (rs[2] + rs[3]);
+          for (int n = 0; n < kNQ; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+              const float p0 = __builtin_amdgcn_exp2f(fmaf(sacc[kb][n][i], scale_log2, -m_run[n]));
+              const float p1 = __builtin_amdgcn_exp2f(fmaf(sacc[kb][n][i + 1], scale_log2, -m_run[n]));
+              pb[kb >> 1][n][2 * (kb & 1) + (i >> 1)] = pack_bf2(p0, p1);
+            }
       }
     }
     // before an even phase 2(t+1): K(t+1) and V(t) (issued kRing - 1 issues ago by their group)
@@ -574,7 +607,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   }
 
   wait_vm_lds<0>();  // no tile load may land in LDS after the workgroup ends
-  store_rows<D>(oacc, l_run, qr, q1, gate, g_row, head, out, o_row, o_head, g);
+  store_rows<D>(oacc, l_run, q0 + wave * 32, q1, gate, g_row, head, out, o_row, o_head, l16, g);
 }
 
 template <int D>
