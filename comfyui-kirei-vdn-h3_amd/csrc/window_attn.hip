@@ -206,10 +206,25 @@ struct RowNorm {
   }
 };
 
-constexpr int kPrepassHeads = 10;  // heads per pre-pass workgroup (they share its rows' RoPE matrices);
-                                   // 10 measured 4% faster than 8 at 40 heads, 4, 5 and 20 no better
+// Heads per pre-pass workgroup. Without RoPE a workgroup has nothing to share between heads: one each
+// (8,296 x 40 x 128: 70 us against 95 with ten, 40,688: 320 against 350, 1,808: 15 against 26). With RoPE the
+// heads of a workgroup share its rows' matrices (about three heads' worth of work to load), against rounds
+// of workgroups over the 512 places (two per CU); up to 256 workgroups have a CU each and run about a quarter
+// faster. 40,688 rows so take 10 heads (519 us; 5: 522, 4: 538, 1: 680), 8,296 rows 6 (120 us; 10: 153, 5: 132,
+// 1: 148) and 1,808 rows 3 (27 us; 10: 46, 4: 31, 1: 34).
+int prepass_heads(int blocks, int heads, bool rope) {
+  if (!rope) return 1;
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int h = 1; h <= 10 && h <= heads; ++h) {
+    const int64_t wgs = (int64_t)blocks * ((heads + h - 1) / h);
+    const int64_t cost = (wgs <= 256 ? 3 : 4 * ((wgs + 511) / 512)) * (h + 3);
+    if (cost < best_cost) best = h, best_cost = cost;
+  }
+  return best;
+}
 
-// Pre-pass of the normalising attention, for the 64 rows [k0, k0 + 64) of up to kPrepassHeads
+// Pre-pass of the normalising attention, for the 64 rows [k0, k0 + 64) of up to group_heads
 // heads: the V^T image chunks of vt_prepass_kernel, the normalised keys kn[head][key][d] and, when q
 // is given, the normalised queries qn[head][row][d] (RowNorm). V tiles alternate between two LDS
 // buffers, so one barrier per head orders the tile's writes before its transposed reads, and the
@@ -220,11 +235,11 @@ __global__ __launch_bounds__(kThreads) void qkv_prepass_kernel(
     const uint16_t *__restrict__ k, int64_t k_row, int64_t k_head, const uint16_t *__restrict__ k_weight, float k_eps,
     const uint16_t *__restrict__ v, int64_t v_row, int64_t v_head, const float *__restrict__ freqs, int64_t f_row,
     int rot, uint16_t *__restrict__ vt, uint16_t *__restrict__ kn, uint16_t *__restrict__ qn, int seq, int s_pad,
-    int heads) {
+    int heads, int group_heads) {
   constexpr int P = D + 8;
   constexpr int CH = D / 8;  // 16-byte chunks per row
   __shared__ __attribute__((aligned(16))) uint16_t tile[2][64 * P];
-  const int h0 = blockIdx.x * kPrepassHeads, h1 = min(heads, h0 + kPrepassHeads);
+  const int h0 = blockIdx.x * group_heads, h1 = min(heads, h0 + group_heads);
   const int k0 = blockIdx.y * 64, tid = threadIdx.x;
   const RowNorm<D, ROPE, kThreads, 64> norm(freqs, f_row, rot, k0, seq, tid);
   for (int head = h0; head < h1; ++head) {
@@ -643,15 +658,16 @@ int launch_qkv_prepass(const uint16_t *q, int64_t q_row, int64_t q_head, const u
   const int s_pad = pad_rows(seq);
   const size_t region = (size_t)heads * D * s_pad;
   uint16_t *vt = static_cast<uint16_t *>(workspace), *kn = vt + region, *qn = vt + 2 * region;
-  const dim3 grid((heads + kPrepassHeads - 1) / kPrepassHeads, s_pad / 64);
+  const int gh = prepass_heads(s_pad / 64, heads, freqs != nullptr);
+  const dim3 grid((heads + gh - 1) / gh, s_pad / 64);
   if (freqs)
     hipLaunchKernelGGL((qkv_prepass_kernel<D, true>), grid, dim3(kThreads), 0, stream, q, q_row, q_head, q_weight,
                        q_eps, k, k_row, k_head, k_weight, k_eps, v, v_row, v_head, freqs, f_row, rot, vt, kn, qn, seq,
-                       s_pad, heads);
+                       s_pad, heads, gh);
   else
     hipLaunchKernelGGL((qkv_prepass_kernel<D, false>), grid, dim3(kThreads), 0, stream, q, q_row, q_head, q_weight,
                        q_eps, k, k_row, k_head, k_weight, k_eps, v, v_row, v_head, freqs, f_row, rot, vt, kn, qn, seq,
-                       s_pad, heads);
+                       s_pad, heads, gh);
   return check_launch("window qkv_prepass");
 }
 

@@ -45,11 +45,22 @@ CASES = [(128, None, False), (64, None, False), (128, 128, False), (128, 64, Tru
 @pytest.mark.parametrize("dim,rot,shared", CASES)
 @pytest.mark.parametrize("with_queries", [False, True])
 def test_qkv_prepass_matches_qk_pass(device, dim, rot, shared, with_queries):
+    _check_prepass(device, dim, rot, shared, with_queries, 1000, 3)
+
+
+# sizes whose heads split into groups of 1, 3, 6 and 10 per workgroup, the last group short, and one row
+@pytest.mark.parametrize("seq,heads", [(1, 1), (1808, 38), (8296, 39), (16007, 56)])
+@pytest.mark.parametrize("rot", [None, 128])
+def test_qkv_prepass_head_groups(device, seq, heads, rot):
+    _check_prepass(device, 128, rot, False, True, seq, heads)
+
+
+def _check_prepass(device, dim, rot, shared, with_queries, seq, heads):
     from vdn_h3_amd import _lib
     from vdn_h3_amd.hybrid import normalise_qk
     from vdn_h3_amd.window import rope_table
 
-    seq, heads, q_eps, k_eps = 1000, 3, 1e-6, 1e-5
+    q_eps, k_eps = 1e-6, 1e-5
     if rot is not None:  # with RoPE the q/k pass takes one epsilon for both
         q_eps = k_eps
     print(f"case qkv_prepass D={dim} rot={rot} shared={shared} queries={with_queries}", flush=True)
