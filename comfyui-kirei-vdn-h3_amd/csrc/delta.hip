@@ -34,7 +34,7 @@ __device__ __forceinline__ f32x16_t mfma_f32_32x32x2(float a, float b, f32x16_t 
 }
 
 // ---------------------------------------------------------------------------------------
-// frame statistics. grid = frames * heads, 256 threads. Tokens are consumed in tiles of 32,
+// frame statistics. One workgroup of 256 threads per (frame, head). Tokens are consumed in tiles of 32,
 // stored transposed ([d][t]) in LDS so both MFMA operands read 8 consecutive tokens; the LDS
 // tiles are double-buffered (one barrier per tile) and each tile's raw k / v / beta are loaded
 // into registers while the previous tile's features are formed and multiplied.
@@ -45,20 +45,31 @@ __device__ __forceinline__ f32x16_t mfma_f32_32x32x2(float a, float b, f32x16_t 
 // AB: A in bf16 as the reference computes it with a_fp32=False (vdn_h3/branch.py:238-240):
 // S = bf16(hi^T k~) (the bf16 product of bf16(k~ * beta) and k~, fp32 accumulation), then
 // 0.5 (S + S^T) in fp32; the lo half and its MFMAs are skipped.
-template <int D, bool KF, bool VF, bool AB>
-__global__ __launch_bounds__(256, 2) void frame_stats_kernel(const uint16_t *__restrict__ k, int64_t k_row,
-                                                             int64_t k_head, const uint16_t *__restrict__ v,
-                                                             int64_t v_row, int64_t v_head,
-                                                             const uint16_t *__restrict__ beta, int64_t beta_row,
-                                                             int T, int heads, float *__restrict__ A_out,
-                                                             float *__restrict__ B_out) {
-  constexpr int TT = 32, P = TT + 8, CH = D / 8, NB = D / 64;
-  constexpr int TILE = D * P;
-  constexpr int BUF_BYTES = 4 * TILE * 2, SYM_BYTES = D * (D + 1) * 4;
-  constexpr int LDS_BYTES = 2 * BUF_BYTES > SYM_BYTES ? 2 * BUF_BYTES : SYM_BYTES;
-  __shared__ __attribute__((aligned(16))) uint8_t smem[LDS_BYTES];
+struct StatsJob {
+  const uint16_t *k, *v, *beta;
+  int64_t k_row, k_head, v_row, v_head, beta_row;
+  int T;
+  float *A, *B;
+};
 
-  const int fh = blockIdx.x, f = fh / heads, h = fh - f * heads;
+template <int D>
+struct StatsTile {
+  static constexpr int TT = 32, P = TT + 8, TILE = D * P;
+  static constexpr int BUF_BYTES = 4 * TILE * 2, SYM_BYTES = D * (D + 1) * 4;
+  static constexpr int LDS_BYTES = 2 * BUF_BYTES > SYM_BYTES ? 2 * BUF_BYTES : SYM_BYTES;
+};
+
+template <int D, bool KF, bool VF, bool AB>
+__device__ __forceinline__ void frame_stats(const StatsJob &job, int fh, int heads, uint8_t *smem) {
+  using Tile = StatsTile<D>;
+  constexpr int TT = Tile::TT, P = Tile::P, CH = D / 8, NB = D / 64, TILE = Tile::TILE, BUF_BYTES = Tile::BUF_BYTES;
+  const uint16_t *__restrict__ k = job.k, *__restrict__ v = job.v, *__restrict__ beta = job.beta;
+  const int64_t k_row = job.k_row, k_head = job.k_head, v_row = job.v_row, v_head = job.v_head,
+                beta_row = job.beta_row;
+  const int T = job.T;
+  float *__restrict__ A_out = job.A, *__restrict__ B_out = job.B;
+
+  const int f = fh / heads, h = fh - f * heads;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int wm = (wave >> 1) * 32 * NB, wn = (wave & 1) * 32 * NB;
   const int p = tid / CH, c = tid % CH;  // loader: token pair p, 16-byte chunk c of the row
@@ -195,6 +206,17 @@ __global__ __launch_bounds__(256, 2) void frame_stats_kernel(const uint16_t *__r
   }
 }
 
+// TEXT: the first text_blocks workgroups take a second job on raw k / v (the text rows, one "frame" per head):
+// alone those 40 workgroups left most of the chip idle for 97 us at 512 text rows x 40 heads x 128.
+template <int D, bool KF, bool VF, bool AB, bool TEXT>
+__global__ __launch_bounds__(256, 2) void frame_stats_kernel(const StatsJob job, const StatsJob text, int text_blocks,
+                                                             int heads) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[StatsTile<D>::LDS_BYTES];
+  const int bid = blockIdx.x;
+  if (TEXT && bid < text_blocks) frame_stats<D, false, false, AB>(text, bid, heads, smem);
+  else frame_stats<D, KF, VF, AB>(job, bid - text_blocks, heads, smem);
+}
+
 // ---------------------------------------------------------------------------------------
 // factor. grid = n matrices, 256 threads. M = (I + A)^-1 by the symmetric sweep operator: the
 // working matrix S starts as I + A and is swept on pivots k = 0 .. D-1,
@@ -206,17 +228,31 @@ __global__ __launch_bounds__(256, 2) void frame_stats_kernel(const uint16_t *__r
 // S in registers (a 16 x 16 grid of sub-blocks); column k of each step is broadcast through a
 // double-buffered LDS line (one barrier per pivot). Then Phi = diag(alpha) M from registers and
 // J = B M on v_mfma_f32_32x32x2_f32.
+//
+// The pivots are a chain of barriers and LDS round trips (about 1500 cycles each), so what counts is how many
+// matrices a CU works on at once: M is staged for J in halves of 64 columns, 34 KB of LDS instead of 67, and the
+// registers stay within 128, four workgroups per CU instead of two: 1,400 matrices of 128 x 128 in 210 us instead
+// of 260. A launch takes up to two jobs (the video frames and the text state, whose 40 matrices alone cost a
+// whole chain, 68 us).
+struct FactorJob {
+  const float *A, *B, *alpha;
+  float *Phi, *J;
+  float j_scale;
+  int *info;
+};
+
 template <int D>
-__global__ __launch_bounds__(256) void factor_kernel(const float *__restrict__ A, const float *__restrict__ B,
-                                                     const float *__restrict__ alpha, float *__restrict__ Phi,
-                                                     float *__restrict__ J, float j_scale, int *__restrict__ info) {
-  constexpr int SB = D / 16, PITCH = D + 1, NBW = D / 64;  // NBW: 32x32 blocks per wave side
+__global__ __launch_bounds__(256, 4) void factor_kernel(const FactorJob job0, const FactorJob job1, int n0) {
+  constexpr int SB = D / 16, HC = 64, PITCH = HC + 1;  // HC: columns of M staged at a time
+  constexpr int NJ = D == 128 ? 2 : 1;                 // 32x32 blocks of J per wavefront and half
   __shared__ float Lb[D * PITCH];
   __shared__ __attribute__((aligned(16))) float bcast[2][D];
-  const int mat = blockIdx.x, tid = threadIdx.x;
+  const bool first = (int)blockIdx.x < n0;
+  const FactorJob &job = first ? job0 : job1;
+  const int mat = first ? blockIdx.x : blockIdx.x - n0, tid = threadIdx.x;
   const int ib = tid >> 4, kb0 = tid & 15;  // sub-block row / column of this thread
   const int i0 = ib * SB, k0 = kb0 * SB;
-  const float *Am = A + (int64_t)mat * D * D;
+  const float *__restrict__ Am = job.A + (int64_t)mat * D * D;
 
   float S[SB][SB];
 #pragma unroll
@@ -262,110 +298,144 @@ __global__ __launch_bounds__(256) void factor_kernel(const float *__restrict__ A
       }
     }
   }
-  if (tid == 0) info[mat] = fail;
+  if (tid == 0) job.info[mat] = fail;
 
-  // M = -S: Phi = diag(alpha) M straight from registers, M into LDS for J = B M
-  float *Pm = Phi ? Phi + (int64_t)mat * D * D : nullptr;
-  const float *al = alpha ? alpha + (int64_t)mat * D : nullptr;
+  // M = -S: Phi = diag(alpha) M straight from registers
+  if (job.Phi) {
+    float *Pm = job.Phi + (int64_t)mat * D * D;
+    const float *al = job.alpha ? job.alpha + (int64_t)mat * D : nullptr;
 #pragma unroll
-  for (int a = 0; a < SB; ++a) {
-    const float sa = al ? -al[i0 + a] : -1.f;
+    for (int a = 0; a < SB; ++a) {
+      const float sa = al ? -al[i0 + a] : -1.f;
 #pragma unroll
-    for (int c = 0; c < SB; ++c) {
-      Lb[(i0 + a) * PITCH + k0 + c] = -S[a][c];
-      if (Pm) Pm[(i0 + a) * D + k0 + c] = sa * S[a][c];
+      for (int c = 0; c < SB; ++c) Pm[(i0 + a) * D + k0 + c] = sa * S[a][c];
     }
   }
-  __syncthreads();
+  // J = B M, HC columns at a time: lane group g contracts over k in [g*D/2, (g+1)*D/2); B rows stream from memory
   const int wave = tid >> 6, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-  const int wm = (wave >> 1) * 32 * NBW, wn = (wave & 1) * 32 * NBW;
-  f32x16_t acc[NBW][NBW];
-
-  // J = B Minv: lane group g contracts over k in [g*D/2, (g+1)*D/2); B rows stream from memory
-  const float *Bm = B + (int64_t)mat * D * D;
+  const int wm = D == 128 ? 32 * wave : 32 * (wave >> 1), wn = D == 128 ? 0 : 32 * (wave & 1);
+  const float *Brow = job.B + (int64_t)mat * D * D + (wm + l32) * D + g * (D / 2);
+  float *Jm = job.J + (int64_t)mat * D * D;
+#pragma unroll 1
+  for (int c0 = 0; c0 < D; c0 += HC) {
+    if (c0) __syncthreads();  // the previous half has been read
+    if (k0 >= c0 && k0 < c0 + HC) {
 #pragma unroll
-  for (int i = 0; i < NBW; ++i)
+      for (int a = 0; a < SB; ++a)
 #pragma unroll
-    for (int j = 0; j < NBW; ++j) acc[i][j] = f32x16_t{};
-  for (int s0 = 0; s0 < D / 2; s0 += 4) {
-    f32x4_t brow[NBW];
-#pragma unroll
-    for (int i = 0; i < NBW; ++i)
-      brow[i] = *reinterpret_cast<const f32x4_t *>(Bm + (wm + 32 * i + l32) * D + g * (D / 2) + s0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int kappa = g * (D / 2) + s0 + e;
-      float bv[NBW];
-#pragma unroll
-      for (int j = 0; j < NBW; ++j) bv[j] = Lb[kappa * PITCH + wn + 32 * j + l32];
-#pragma unroll
-      for (int i = 0; i < NBW; ++i)
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) acc[i][j] = mfma_f32_32x32x2(brow[i][e], bv[j], acc[i][j]);
+        for (int c = 0; c < SB; ++c) Lb[(i0 + a) * PITCH + k0 - c0 + c] = -S[a][c];
     }
-  }
-  float *Jm = J + (int64_t)mat * D * D;
+    __syncthreads();
+    f32x16_t acc[NJ];
 #pragma unroll
-  for (int i = 0; i < NBW; ++i)
+    for (int j = 0; j < NJ; ++j) acc[j] = f32x16_t{};
+#pragma unroll 4
+    for (int s0 = 0; s0 < D / 2; s0 += 4) {
+      const f32x4_t brow = *reinterpret_cast<const f32x4_t *>(Brow + s0);
 #pragma unroll
-    for (int j = 0; j < NBW; ++j)
+      for (int e = 0; e < 4; ++e) {
+        const int kappa = g * (D / 2) + s0 + e;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          acc[j] = mfma_f32_32x32x2(brow[e], Lb[kappa * PITCH + wn + 32 * j + l32], acc[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), n = wn + 32 * j + l32;
-        Jm[m * D + n] = j_scale * acc[i][j][r];
+        const int m = wm + 8 * (r >> 2) + 4 * g + (r & 3), n = c0 + wn + 32 * j + l32;
+        Jm[m * D + n] = job.j_scale * acc[j][r];
       }
+  }
 }
 
 // ---------------------------------------------------------------------------------------
-// scan. grid = heads * 2 directions * D/32 row blocks; D/32 wavefronts, wavefront w owns state
+// scan. One workgroup per (head, direction, 32-row block); D/32 wavefronts, wavefront w owns state
 // columns [32w, 32w+32). The state is kept transposed, X = P^T, so the 32x32 accumulator of
 // one step (lane = state row) is the next step's B operand after one LDS exchange:
 //   X_f = Phi_f^T X_{f-1} + J_f^T
+// The steps are a chain, their operands are not: a step loads the next one's Phi and J into a second register
+// set, eight loads after every eight products (all issued before the products they exceed the 63 operations
+// a wait can count, and the products waited for all of them; one load after each product was 30% slower).
+// Contraction index kappa = 8 (s / 4) + 4 g + s % 4 belongs to product s and lane group g, and the state lies
+// in LDS by (g, row, s), so a lane reads and writes it 16 bytes at a time. 40 heads of 128, 35 frames: 260 ->
+// 219 us (176 without the loads: the 64 CUs that hold two of the 320 workgroups set the time); 8 heads, 11
+// frames: 53 -> 34 us; 13 heads of 64, 70 frames: 163 -> 94 us.
 template <int D>
 __global__ __launch_bounds__(64 * (D / 32)) void scan_kernel(const float *__restrict__ Phi, const float *__restrict__ J,
                                                              const float *__restrict__ init,
                                                              float *__restrict__ prefix, float *__restrict__ suffix,
-                                                             int F, int heads) {
-  constexpr int NRB = D / 32, PITCH = 32 + 4;
-  __shared__ float St[2][D * PITCH];
-  const int bid = blockIdx.x;
-  const int rb = bid % NRB, dir = (bid / NRB) & 1, h = bid / (2 * NRB);
+                                                             int F, int heads, int per_xcd) {
+  constexpr int NRB = D / 32, NS = D / 2, PITCH = NS + 4;
+  __shared__ __attribute__((aligned(16))) float St[2][2][32 * PITCH];  // [buffer][g][row][s]
+  // workgroups are dealt round-robin over the 8 XCDs: XCD x takes items x per_xcd .. + per_xcd, so the row blocks of
+  // a (head, direction), which read the same Phi, share its L2
+  const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (item >= heads * 2 * NRB) return;
+  const int rb = item % NRB, dir = (item / NRB) & 1, h = item / (2 * NRB);
   const int tid = threadIdx.x, cb = tid >> 6, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int r0 = rb * 32;
   for (int e = tid; e < D * 32; e += 64 * NRB) {
     const int c = e >> 5, r = e & 31;
-    St[0][c * PITCH + r] = init ? init[((int64_t)h * D + r0 + r) * D + c] : 0.f;
+    St[0][(c >> 2) & 1][r * PITCH + 4 * (c >> 3) + (c & 3)] =
+        init ? init[((int64_t)h * D + r0 + r) * D + c] : 0.f;
   }
   __syncthreads();
   float *out = dir == 0 ? prefix : suffix;
-  int cur = 0;
-  for (int step = 0; step < F; ++step) {
-    const int f = dir == 0 ? step : F - 1 - step;
-    const int64_t base = ((int64_t)f * heads + h) * D * D;
-    const float *Pf = Phi + base;
+  const int64_t hd2 = (int64_t)h * D * D, frame = (int64_t)heads * D * D;
+  const uint32_t phi_lane = 4 * g * D + 32 * cb + l32;                      // + (s % 4) D
+  const int64_t row_lane = hd2 + (int64_t)(r0 + l32) * D + 32 * cb + 4 * g;  // + 8 i4: J and the output
+  auto frame_of = [&](int step) __device__ { return (dir == 0 ? step : F - 1 - step) * frame; };
+  struct Operands {
+    float phi[NS];
+    f32x4_t j[4];
+  };
+  // one step on `o`, loading the next step's operands into `n` (the last step loads its own again, unused)
+  auto advance = [&](int step, const Operands &o, Operands &n) __device__ {
+    const float *X = St[step & 1][g] + l32 * PITCH;
+    f32x4_t x[NS / 4];
+#pragma unroll
+    for (int s4 = 0; s4 < NS / 4; ++s4) x[s4] = *reinterpret_cast<const f32x4_t *>(X + 4 * s4);
+    const int64_t next = frame_of(min(step + 1, F - 1));
+    const float *Pn = Phi + next + hd2, *Jn = J + next + row_lane;
     f32x16_t acc = f32x16_t{};
-#pragma unroll 16
-    for (int s = 0; s < D / 2; ++s) {
-      const int kappa = 2 * s + g;
-      acc = mfma_f32_32x32x2(Pf[kappa * D + 32 * cb + l32], St[cur][kappa * PITCH + l32], acc);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      acc = mfma_f32_32x32x2(o.phi[s], x[s >> 2][s & 3], acc);
+      n.phi[s] = (Pn + 8 * (s >> 2) * D)[phi_lane + (s & 3) * D];
+      if ((s & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
-    const float *Jr = J + base + (int64_t)(r0 + l32) * D;
-    float *Or = out + base + (int64_t)(r0 + l32) * D;
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) n.j[i4] = *reinterpret_cast<const f32x4_t *>(Jn + 8 * i4);
+    float *Or = out + frame_of(step) + row_lane;
+    float *Y = St[(step & 1) ^ 1][g] + l32 * PITCH + 16 * cb;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
-      const int c0 = 32 * cb + 8 * i4 + 4 * g;
-      const f32x4_t jv = *reinterpret_cast<const f32x4_t *>(Jr + c0);
-      f32x4_t o;
+      f32x4_t r;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        o[e] = acc[4 * i4 + e] + jv[e];
-        St[cur ^ 1][(c0 + e) * PITCH + l32] = o[e];
-      }
-      *reinterpret_cast<f32x4_t *>(Or + c0) = o;
+      for (int e = 0; e < 4; ++e) r[e] = acc[4 * i4 + e] + o.j[i4][e];
+      *reinterpret_cast<f32x4_t *>(Y + 4 * i4) = r;
+      *reinterpret_cast<f32x4_t *>(Or + 8 * i4) = r;
     }
-    __syncthreads();
-    cur ^= 1;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the state is in LDS; loads and stores stay in flight
+    bare_barrier();
+  };
+  Operands o0, o1;
+  {
+    const float *P0 = Phi + frame_of(0) + hd2, *J0 = J + frame_of(0) + row_lane;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) o0.phi[s] = (P0 + 8 * (s >> 2) * D)[phi_lane + (s & 3) * D];
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) o0.j[i4] = *reinterpret_cast<const f32x4_t *>(J0 + 8 * i4);
   }
+  int step = 0;
+#pragma unroll 1
+  for (; step + 1 < F; step += 2) {
+    advance(step, o0, o1);
+    advance(step + 1, o1, o0);
+  }
+  if (step < F) advance(step, o0, o1);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -827,52 +897,107 @@ using vdnh3::check_dim;
 using vdnh3::check_launch;
 using vdnh3::set_error;
 
+namespace vdnh3 {
+namespace {
+
+int check_stats_job(const vdnh3_frame_stats_job &j) {
+  VDNH3_HOST_CHECK(j.k && j.v && j.beta && j.A && j.B && j.frames > 0 && j.tokens > 0, VDNH3_ERR_INVALID,
+                   "frame_stats: empty or null operand");
+  VDNH3_HOST_CHECK(j.k_row % 8 == 0 && j.k_head % 8 == 0 && j.v_row % 8 == 0 && j.v_head % 8 == 0 &&
+                       reinterpret_cast<uintptr_t>(j.k) % 16 == 0 && reinterpret_cast<uintptr_t>(j.v) % 16 == 0,
+                   VDNH3_ERR_INVALID, "frame_stats: k/v must be 16-byte aligned with strides multiple of 8");
+  VDNH3_HOST_CHECK((j.features & ~7) == 0, VDNH3_ERR_INVALID, "frame_stats: unknown feature flags %d", j.features);
+  return VDNH3_OK;
+}
+
+StatsJob stats_job(const vdnh3_frame_stats_job &j) {
+  return StatsJob{j.k, j.v, j.beta, j.k_row, j.k_head, j.v_row, j.v_head, j.beta_row, j.tokens, j.A, j.B};
+}
+
+// `job`, and with `text` (raw features, the same bit 2) a second one in the same launch
+template <int D, bool KF, bool VF, bool AB>
+void launch_stats(const vdnh3_frame_stats_job &job, const vdnh3_frame_stats_job *text, int heads, hipStream_t s) {
+  const StatsJob main = stats_job(job);
+  if (text)
+    hipLaunchKernelGGL((frame_stats_kernel<D, KF, VF, AB, true>), dim3((job.frames + text->frames) * heads), dim3(256),
+                       0, s, main, stats_job(*text), text->frames * heads, heads);
+  else
+    hipLaunchKernelGGL((frame_stats_kernel<D, KF, VF, AB, false>), dim3(job.frames * heads), dim3(256), 0, s, main,
+                       main, 0, heads);
+}
+
+template <int D>
+void launch_stats_dim(const vdnh3_frame_stats_job &job, const vdnh3_frame_stats_job *text, int heads, hipStream_t s) {
+  switch (job.features) {
+    case 0: return launch_stats<D, 0, 0, 0>(job, text, heads, s);
+    case 1: return launch_stats<D, 1, 0, 0>(job, text, heads, s);
+    case 2: return launch_stats<D, 0, 1, 0>(job, text, heads, s);
+    case 3: return launch_stats<D, 1, 1, 0>(job, text, heads, s);
+    case 4: return launch_stats<D, 0, 0, 1>(job, text, heads, s);
+    case 5: return launch_stats<D, 1, 0, 1>(job, text, heads, s);
+    case 6: return launch_stats<D, 0, 1, 1>(job, text, heads, s);
+    default: return launch_stats<D, 1, 1, 1>(job, text, heads, s);
+  }
+}
+
+}  // namespace
+}  // namespace vdnh3
+
+extern "C" int vdnh3_frame_stats_batch(const vdnh3_frame_stats_job *jobs, int n_jobs, int heads, int head_dim,
+                                       void *stream) {
+  int rc = check_dim(head_dim);
+  if (rc) return rc;
+  VDNH3_HOST_CHECK(jobs && n_jobs >= 1 && n_jobs <= 2 && heads > 0, VDNH3_ERR_INVALID,
+                   "frame_stats: 1 or 2 jobs, got %d", n_jobs);
+  for (int i = 0; i < n_jobs; ++i)
+    if ((rc = vdnh3::check_stats_job(jobs[i]))) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // one launch takes a second job on raw k / v with the first one's A precision; any other pair takes two
+  const bool fused = n_jobs == 2 && (jobs[1].features & 3) == 0 && (jobs[0].features & 4) == (jobs[1].features & 4);
+  for (int i = 0; i < (fused ? 1 : n_jobs); ++i) {
+    const vdnh3_frame_stats_job *text = fused ? jobs + 1 : nullptr;
+    if (head_dim == 128) vdnh3::launch_stats_dim<128>(jobs[i], text, heads, s);
+    else vdnh3::launch_stats_dim<64>(jobs[i], text, heads, s);
+    if ((rc = check_launch("frame_stats"))) return rc;
+  }
+  return VDNH3_OK;
+}
+
 extern "C" int vdnh3_frame_stats(const uint16_t *k, int64_t k_row, int64_t k_head, const uint16_t *v,
                                  int64_t v_row, int64_t v_head, int features, const uint16_t *beta,
                                  int64_t beta_row, int frames, int tokens, int heads, int head_dim, float *A,
                                  float *B, void *stream) {
+  const vdnh3_frame_stats_job job{k, k_row, k_head, v, v_row, v_head, features, beta, beta_row, frames, tokens, A, B};
+  return vdnh3_frame_stats_batch(&job, 1, heads, head_dim, stream);
+}
+
+extern "C" int vdnh3_delta_factor_batch(const vdnh3_delta_factor_job *jobs, int n_jobs, int head_dim, void *stream) {
   int rc = check_dim(head_dim);
   if (rc) return rc;
-  VDNH3_HOST_CHECK(k && v && beta && A && B && frames > 0 && tokens > 0 && heads > 0, VDNH3_ERR_INVALID,
-                   "frame_stats: empty or null operand");
-  VDNH3_HOST_CHECK(k_row % 8 == 0 && k_head % 8 == 0 && v_row % 8 == 0 && v_head % 8 == 0 &&
-                       reinterpret_cast<uintptr_t>(k) % 16 == 0 && reinterpret_cast<uintptr_t>(v) % 16 == 0,
-                   VDNH3_ERR_INVALID, "frame_stats: k/v must be 16-byte aligned with strides multiple of 8");
-  VDNH3_HOST_CHECK((features & ~7) == 0, VDNH3_ERR_INVALID, "frame_stats: unknown feature flags %d", features);
+  VDNH3_HOST_CHECK(jobs && n_jobs >= 1 && n_jobs <= 2, VDNH3_ERR_INVALID, "delta_factor: 1 or 2 jobs, got %d", n_jobs);
+  vdnh3::FactorJob fj[2] = {};
+  int total = 0;
+  for (int i = 0; i < n_jobs; ++i) {
+    const vdnh3_delta_factor_job &j = jobs[i];
+    VDNH3_HOST_CHECK(j.A && j.B && j.jay && j.info && j.n > 0, VDNH3_ERR_INVALID,
+                     "delta_factor: empty or null operand");
+    VDNH3_HOST_CHECK(reinterpret_cast<uintptr_t>(j.B) % 16 == 0, VDNH3_ERR_INVALID,
+                     "delta_factor: B must be 16-byte aligned");
+    fj[i] = vdnh3::FactorJob{j.A, j.B, j.alpha, j.phi, j.jay, j.jay_scale, j.info};
+    total += j.n;
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(frames * heads);
-#define VDNH3_FS(D, KF, VF, AB)                                                                                \
-  if (head_dim == D && (features & 1) == KF && ((features >> 1) & 1) == VF && ((features >> 2) & 1) == AB)   \
-    hipLaunchKernelGGL((vdnh3::frame_stats_kernel<D, KF, VF, AB>), grid, dim3(256), 0, s, k, k_row, k_head, v, \
-                       v_row, v_head, beta, beta_row, tokens, heads, A, B);
-#define VDNH3_FS_D(D)    \
-  VDNH3_FS(D, 0, 0, 0)   \
-  VDNH3_FS(D, 1, 0, 0)   \
-  VDNH3_FS(D, 0, 1, 0)   \
-  VDNH3_FS(D, 1, 1, 0)   \
-  VDNH3_FS(D, 0, 0, 1)   \
-  VDNH3_FS(D, 1, 0, 1)   \
-  VDNH3_FS(D, 0, 1, 1)   \
-  VDNH3_FS(D, 1, 1, 1)
-  VDNH3_FS_D(128)
-  VDNH3_FS_D(64)
-#undef VDNH3_FS_D
-#undef VDNH3_FS
-  return check_launch("frame_stats");
+  if (head_dim == 128)
+    hipLaunchKernelGGL(vdnh3::factor_kernel<128>, dim3(total), dim3(256), 0, s, fj[0], fj[1], jobs[0].n);
+  else
+    hipLaunchKernelGGL(vdnh3::factor_kernel<64>, dim3(total), dim3(256), 0, s, fj[0], fj[1], jobs[0].n);
+  return check_launch("delta_factor");
 }
 
 extern "C" int vdnh3_delta_factor(const float *A, const float *B, const float *alpha, float *phi, float *jay,
                                   float jay_scale, int32_t *info, int n, int head_dim, void *stream) {
-  int rc = check_dim(head_dim);
-  if (rc) return rc;
-  VDNH3_HOST_CHECK(A && B && jay && info && n > 0, VDNH3_ERR_INVALID, "delta_factor: empty or null operand");
-  VDNH3_HOST_CHECK(reinterpret_cast<uintptr_t>(B) % 16 == 0, VDNH3_ERR_INVALID, "delta_factor: B must be 16-byte aligned");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (head_dim == 128)
-    hipLaunchKernelGGL(vdnh3::factor_kernel<128>, dim3(n), dim3(256), 0, s, A, B, alpha, phi, jay, jay_scale, info);
-  else
-    hipLaunchKernelGGL(vdnh3::factor_kernel<64>, dim3(n), dim3(256), 0, s, A, B, alpha, phi, jay, jay_scale, info);
-  return check_launch("delta_factor");
+  const vdnh3_delta_factor_job job{A, B, alpha, phi, jay, jay_scale, info, n};
+  return vdnh3_delta_factor_batch(&job, 1, head_dim, stream);
 }
 
 extern "C" int vdnh3_sana_factor(const float *A, const float *B, const float *alpha, float *phi, float *jay,
@@ -895,11 +1020,14 @@ extern "C" int vdnh3_delta_scan(const float *phi, const float *jay, const float 
   VDNH3_HOST_CHECK(phi && jay && prefix && suffix && frames > 0 && heads > 0, VDNH3_ERR_INVALID,
                    "delta_scan: empty or null operand");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(heads * 2 * (head_dim / 32));
+  const int per_xcd = (heads * 2 * (head_dim / 32) + 7) / 8;
+  const dim3 grid(8 * per_xcd);
   if (head_dim == 128)
-    hipLaunchKernelGGL(vdnh3::scan_kernel<128>, grid, dim3(256), 0, s, phi, jay, init, prefix, suffix, frames, heads);
+    hipLaunchKernelGGL(vdnh3::scan_kernel<128>, grid, dim3(256), 0, s, phi, jay, init, prefix, suffix, frames, heads,
+                       per_xcd);
   else
-    hipLaunchKernelGGL(vdnh3::scan_kernel<64>, grid, dim3(128), 0, s, phi, jay, init, prefix, suffix, frames, heads);
+    hipLaunchKernelGGL(vdnh3::scan_kernel<64>, grid, dim3(128), 0, s, phi, jay, init, prefix, suffix, frames, heads,
+                       per_xcd);
   return check_launch("delta_scan");
 }
 

@@ -105,6 +105,23 @@ def frame_statistics_raw(k_raw: torch.Tensor, v_raw: torch.Tensor, beta: torch.T
     the bf16 product of ``bf16(k~ * beta)`` and ``k~``, rounded to bf16, then symmetrised.
     ``out=(A, B)``: contiguous fp32 ``[F, H, D, D]`` tensors (e.g. frame slices of larger ones) to write into.
     """
+    job, heads, dim, device, out, held = _stats_job(k_raw, v_raw, beta, num_frames, tokens_per_frame, k_features,
+                                                    v_features, a_fp32, out)
+    rc = _lib.lib().vdnh3_frame_stats_batch(ctypes.addressof(job), 1, heads, dim, _lib.stream_handle(device))
+    _lib.check(rc, "vdnh3_frame_stats_batch")
+    del held
+    return out
+
+
+class _StatsJob(ctypes.Structure):
+    """``vdnh3_frame_stats_job`` (include/vdnh3.h)."""
+    _fields_ = [("k", ctypes.c_void_p), ("k_row", ctypes.c_int64), ("k_head", ctypes.c_int64),
+                ("v", ctypes.c_void_p), ("v_row", ctypes.c_int64), ("v_head", ctypes.c_int64),
+                ("features", ctypes.c_int), ("beta", ctypes.c_void_p), ("beta_row", ctypes.c_int64),
+                ("frames", ctypes.c_int), ("tokens", ctypes.c_int), ("A", ctypes.c_void_p), ("B", ctypes.c_void_p)]
+
+
+def _stats_job(k_raw, v_raw, beta, num_frames, tokens_per_frame, k_features, v_features, a_fp32, out):
     if k_raw.shape != v_raw.shape or k_raw.ndim != 3:
         raise ValueError("key and value must share shape [rows, heads, dim]")
     rows, heads, dim = k_raw.shape
@@ -127,12 +144,25 @@ def frame_statistics_raw(k_raw: torch.Tensor, v_raw: torch.Tensor, beta: torch.T
             if t.shape != (num_frames, heads, dim, dim) or t.dtype != torch.float32 or not t.is_contiguous():
                 raise ValueError(f"out must hold two contiguous fp32 [{num_frames}, {heads}, {dim}, {dim}] tensors")
     flags = int(bool(k_features)) | (int(bool(v_features)) << 1) | (int(not a_fp32) << 2)
-    rc = _lib.lib().vdnh3_frame_stats(_lib.ptr(k_raw), k_raw.stride(0), k_raw.stride(1), _lib.ptr(v_raw),
-                                      v_raw.stride(0), v_raw.stride(1), flags, _lib.ptr(beta), beta.stride(0),
-                                      num_frames, tokens_per_frame, heads, dim, _lib.ptr(a), _lib.ptr(b),
-                                      _lib.stream_handle(device))
-    _lib.check(rc, "vdnh3_frame_stats")
-    return a, b
+    job = _StatsJob(_lib.ptr(k_raw), k_raw.stride(0), k_raw.stride(1), _lib.ptr(v_raw), v_raw.stride(0),
+                    v_raw.stride(1), flags, _lib.ptr(beta), beta.stride(0), num_frames, tokens_per_frame, _lib.ptr(a),
+                    _lib.ptr(b))
+    return job, heads, dim, device, (a, b), (k_raw, v_raw, beta)
+
+
+def frame_statistics_with_text(k_raw, v_raw, beta, num_frames, tokens_per_frame, text_k, text_v, text_beta, *,
+                               k_features: bool = False, v_features: bool = False, a_fp32: bool = True):
+    """``frame_statistics_raw`` of the video rows and of the raw text rows (as one frame) in one launch:
+    ``((A, B), (text A, text B))``."""
+    video = _stats_job(k_raw, v_raw, beta, num_frames, tokens_per_frame, k_features, v_features, a_fp32, None)
+    text = _stats_job(text_k, text_v, text_beta, 1, text_k.shape[0], False, False, a_fp32, None)
+    if video[1:4] != text[1:4]:
+        raise ValueError("video and text rows must share heads, head dim and device")
+    jobs = (_StatsJob * 2)(video[0], text[0])
+    rc = _lib.lib().vdnh3_frame_stats_batch(ctypes.addressof(jobs), 2, video[1], video[2],
+                                            _lib.stream_handle(video[3]))
+    _lib.check(rc, "vdnh3_frame_stats_batch")
+    return video[4], text[4]
 
 
 class _ConvJob(ctypes.Structure):
@@ -218,13 +248,19 @@ def conv_features_batch(items, num_frames: int, frame_size) -> list:
     return outs
 
 
+class _FactorJob(ctypes.Structure):
+    """``vdnh3_delta_factor_job`` (include/vdnh3.h)."""
+    _fields_ = [("A", ctypes.c_void_p), ("B", ctypes.c_void_p), ("alpha", ctypes.c_void_p), ("phi", ctypes.c_void_p),
+                ("jay", ctypes.c_void_p), ("jay_scale", ctypes.c_float), ("info", ctypes.c_void_p), ("n", ctypes.c_int)]
+
+
 class VdnDelta:
     """``Phi = diag(alpha) (I + A)^-1``, ``J = B (I + A)^-1`` by Cholesky, with deferred SPD checks."""
 
     def __init__(self, tokens_per_frame: int | None = None):
         del tokens_per_frame
 
-    def factor_apply(self, alpha, a_raw, b_raw, *, jay_scale: float = 1.0, need_phi: bool = True):
+    def _job(self, alpha, a_raw, b_raw, jay_scale, need_phi):
         if a_raw.shape != b_raw.shape or a_raw.shape[-1] != a_raw.shape[-2]:
             raise ValueError("A and B must share a square [..., D, D] shape")
         if alpha is not None and alpha.shape != a_raw.shape[:-1]:
@@ -233,16 +269,35 @@ class VdnDelta:
         _dim(dim)
         device = _lib.require_device(a_raw, b_raw, alpha)
         a32, b32 = a_raw.float().contiguous(), b_raw.float().contiguous()
-        n = a32.numel() // (dim * dim)
         phi = torch.empty_like(a32) if need_phi else None
         jay = torch.empty_like(a32)
         info = torch.empty(a32.shape[:-2], dtype=torch.int32, device=device)
         al = None if alpha is None else alpha.float().contiguous()
-        rc = _lib.lib().vdnh3_delta_factor(_lib.ptr(a32), _lib.ptr(b32), _lib.ptr(al), _lib.ptr(phi), _lib.ptr(jay),
-                                           float(jay_scale), _lib.ptr(info), n, dim, _lib.stream_handle(device))
-        _lib.check(rc, "vdnh3_delta_factor")
+        job = _FactorJob(_lib.ptr(a32), _lib.ptr(b32), _lib.ptr(al), _lib.ptr(phi), _lib.ptr(jay), float(jay_scale),
+                         _lib.ptr(info), a32.numel() // (dim * dim))
+        return job, dim, device, phi, jay, info, (a32, b32, al)
+
+    def factor_apply(self, alpha, a_raw, b_raw, *, jay_scale: float = 1.0, need_phi: bool = True):
+        job, dim, device, phi, jay, info, held = self._job(alpha, a_raw, b_raw, jay_scale, need_phi)
+        rc = _lib.lib().vdnh3_delta_factor_batch(ctypes.addressof(job), 1, dim, _lib.stream_handle(device))
+        _lib.check(rc, "vdnh3_delta_factor_batch")
+        del held
         _record_status(info)
         return phi, jay
+
+    def factor_apply_with_text(self, alpha, a_raw, b_raw, text_a, text_b):
+        """``(Phi, J, text J)``: ``factor_apply`` of the frames and of the text rows' statistics (``J`` only, times
+        ``TEXT_STATE_SCALE``) in one launch; the text status is recorded first, as by two calls."""
+        video = self._job(alpha, a_raw, b_raw, 1.0, True)
+        text = self._job(None, text_a, text_b, TEXT_STATE_SCALE, False)
+        if video[1:3] != text[1:3]:
+            raise ValueError("video and text statistics must share head dim and device")
+        jobs = (_FactorJob * 2)(video[0], text[0])
+        rc = _lib.lib().vdnh3_delta_factor_batch(ctypes.addressof(jobs), 2, video[1], _lib.stream_handle(video[2]))
+        _lib.check(rc, "vdnh3_delta_factor_batch")
+        _record_status(text[5])
+        _record_status(video[5])
+        return video[3], video[4], text[4]
 
 
 class SanaDelta:

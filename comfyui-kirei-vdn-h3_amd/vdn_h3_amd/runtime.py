@@ -80,7 +80,8 @@ class OptimizedLinearBranch:
     def _backend(self, tokens):
         return _b.DELTA_BACKENDS[self.delta_rule](tokens)
 
-    def _text_state(self, weights, text_x, text_k_raw, text_v_raw, beta=None):
+    def _text_rows(self, weights, text_x, text_k_raw, text_v_raw, beta=None):
+        """``(k, v, beta)`` of the text rows the text state is formed from, or ``None`` without one."""
         if not self.enable_text_state or text_x is None:
             return None
         if text_k_raw is None or text_v_raw is None:
@@ -90,9 +91,30 @@ class OptimizedLinearBranch:
             raise ValueError("text tensors must share a positive sequence length")
         if beta is None:
             beta = _linear.sigmoid_linear(text_x, weights["beta_proj.weight"])
-        a, b = _b.frame_statistics_raw(text_k_raw, text_v_raw, beta, 1, length, a_fp32=self.a_fp32)
+        return text_k_raw, text_v_raw, beta
+
+    def _text_state(self, weights, text_x, text_k_raw, text_v_raw, beta=None):
+        rows = self._text_rows(weights, text_x, text_k_raw, text_v_raw, beta)
+        if rows is None:
+            return None
+        k, v, beta = rows
+        length = k.shape[0]
+        a, b = _b.frame_statistics_raw(k, v, beta, 1, length, a_fp32=self.a_fp32)
         _, jay = self._backend(length).factor_apply(None, a, b, jay_scale=_b.TEXT_STATE_SCALE, need_phi=False)
         return jay[0]
+
+    def _scans(self, alpha, stats, text_stats, tokens_per_frame, text_rows):
+        """``(prefix, suffix, text_state)`` from the frames' statistics and, with a text state, the text rows'."""
+        backend = self._backend(tokens_per_frame)
+        if text_stats is None:
+            return *_b.run_scans_inference(backend, alpha, *stats), None
+        if hasattr(backend, "factor_apply_with_text"):
+            phi, jay, text = backend.factor_apply_with_text(alpha, *stats, *text_stats)
+        else:
+            _, text = self._backend(text_rows).factor_apply(None, *text_stats, jay_scale=_b.TEXT_STATE_SCALE,
+                                                            need_phi=False)
+            phi, jay = backend.factor_apply(alpha, *stats)
+        return *_b.run_scans_from_factors(phi, jay, text[0]), text[0]
 
     def _beta_down_weight(self, weights):
         """``[W_beta; W_down]`` (``[heads + rank, hidden]`` bf16), rebuilt when either weight changes."""
@@ -149,15 +171,20 @@ class OptimizedLinearBranch:
         else:
             k_in, k_feat = self._features(weights, "k", k_raw, num_frames, frame_size)
             v_in, v_feat = self._features(weights, "v", v_raw, num_frames, frame_size)
-        a, b = _b.frame_statistics_raw(k_in, v_in, beta, num_frames, tokens_per_frame, k_features=k_feat,
-                                       v_features=v_feat, a_fp32=self.a_fp32)
+        text = self._text_rows(weights, text_x, text_k_raw, text_v_raw, text_beta)
+        features = dict(k_features=k_feat, v_features=v_feat, a_fp32=self.a_fp32)
+        if text is None:
+            stats, text_stats = _b.frame_statistics_raw(k_in, v_in, beta, num_frames, tokens_per_frame, **features), None
+        else:
+            stats, text_stats = _b.frame_statistics_with_text(k_in, v_in, beta, num_frames, tokens_per_frame, *text,
+                                                              **features)
         del k_in, v_in
         mean = _b.frame_mean(xv, num_frames, tokens_per_frame)
         alpha = _b.alpha_gate(mean, weights["alpha.down.weight"], weights["alpha.up.weight"],
                               weights["alpha.dt_bias"], weights["alpha.A_log"], heads, dim)
-        text_state = self._text_state(weights, text_x, text_k_raw, text_v_raw, text_beta)
-        prefix, suffix = _b.run_scans_inference(self._backend(tokens_per_frame), alpha, a, b, text_state)
-        del a, b
+        prefix, suffix, text_state = self._scans(alpha, stats, text_stats, tokens_per_frame,
+                                                 0 if text is None else text[0].shape[0])
+        del stats, text_stats
         q_in, q_feat = self._features(weights, "q", q_raw, num_frames, frame_size)
         # the output gate's up-projection and sigmoid run inside the readout kernel
         return _b.readout_epilogue(q_in, prefix, suffix, alpha, bounds, weights["norm.weight"], None,

@@ -225,6 +225,24 @@ int vdnh3_frame_stats(const uint16_t *k, int64_t k_row, int64_t k_head, const ui
                       int tokens, int heads, int head_dim, float *A, float *B, void *stream);
 
 /*
+ * One or two such calls over the same heads in one call: the video frames, then the text rows as one frame
+ * (vdn_h3/branch.py:649-670). A second job on raw k / v (features bits 0 and 1 clear) with the first job's bit 2
+ * shares the first one's launch. The results are those of vdnh3_frame_stats per job.
+ */
+typedef struct vdnh3_frame_stats_job {
+  const uint16_t *k;
+  int64_t k_row, k_head;
+  const uint16_t *v;
+  int64_t v_row, v_head;
+  int features;
+  const uint16_t *beta;
+  int64_t beta_row;
+  int frames, tokens;
+  float *A, *B;
+} vdnh3_frame_stats_job;
+int vdnh3_frame_stats_batch(const vdnh3_frame_stats_job *jobs, int n_jobs, int heads, int head_dim, void *stream);
+
+/*
  * K/V (or Q) short convolutions of the branch features (vdn_h3/runtime.py:319-341,
  * vdn_h3/branch.py:443-480, vdn_h3/kernels.py:100-129). x holds frames * grid_h * grid_w rows
  * (frame-major, then row-major over the grid), element (r, h, d) at x[r*x_row + h*x_head + d]:
@@ -264,6 +282,16 @@ int vdnh3_short_conv_batch(const vdnh3_short_conv_job *jobs, int n_jobs, int ker
  */
 int vdnh3_delta_factor(const float *A, const float *B, const float *alpha, float *phi, float *jay,
                        float jay_scale, int32_t *info, int n, int head_dim, void *stream);
+
+/* One or two such calls in one launch; the results are those of vdnh3_delta_factor per job. */
+typedef struct vdnh3_delta_factor_job {
+  const float *A, *B, *alpha;
+  float *phi, *jay;
+  float jay_scale;
+  int32_t *info;
+  int n;
+} vdnh3_delta_factor_job;
+int vdnh3_delta_factor_batch(const vdnh3_delta_factor_job *jobs, int n_jobs, int head_dim, void *stream);
 
 /* SanaDelta.factor_apply (vdn_h3/branch.py:163-177): phi = alpha (I - A/T), jay = jay_scale * (B / sqrt(T)),
  * each fp32 product / difference rounded on its own as the reference's tensor ops do; alpha NULL

@@ -154,6 +154,56 @@ def test_scans(device, text):
     _close(s, ws, 1e-4, 1e-5, "suffix")
 
 
+# one step, odd and even step counts, and item counts (heads x 2 x dim / 32) below, off and at a multiple of 8
+@pytest.mark.parametrize("frames,heads,dim", [(1, 1, 64), (2, 3, 128), (5, 2, 64), (6, 5, 128)])
+def test_scan_steps_and_item_counts(device, frames, heads, dim):
+    from vdn_h3_amd import branch
+
+    print(f"case scan F={frames} H={heads} D={dim}", flush=True)
+    phi = _rand((frames, heads, dim, dim), 91, dim ** -0.5).to(device)
+    jay = _rand((frames, heads, dim, dim), 92).to(device)
+    init = _rand((heads, dim, dim), 93).to(device)
+    got = branch.run_scans_from_factors(phi, jay, init)
+    for out, order in zip(got, (range(frames), reversed(range(frames)))):
+        s, bound = init.double(), init.double().abs()
+        for f in order:
+            s = jay[f].double() + s @ phi[f].double()
+            # fp32 products and sums: at most dim + 1 roundings a step on sums of absolute values
+            bound = jay[f].double().abs() + bound @ phi[f].double().abs()
+            err = (out[f].double() - s).abs()
+            assert bool((err <= frames * (dim + 1) * 2.0 ** -24 * bound).all()), (f, err.max().item())
+
+
+@pytest.mark.parametrize("dim,k_features,v_features,a_fp32,text_rows", [
+    (128, True, True, True, 33), (128, False, False, True, 1), (64, True, False, False, 64), (64, False, True, True, 200)])
+def test_text_state_shares_the_video_launches(device, dim, k_features, v_features, a_fp32, text_rows):
+    """Statistics and factors of the video frames and the text rows in one launch each are the separate calls' bits."""
+    from vdn_h3_amd import branch
+
+    print(f"case text in video launches D={dim}", flush=True)
+    frames, tokens, heads = 3, 70, 3
+    rows = frames * tokens
+    k, v, tk, tv = (_rand((n, heads, dim), i, dtype=torch.bfloat16).to(device)
+                    for i, n in ((71, rows), (72, rows), (73, text_rows), (74, text_rows)))
+    beta, tbeta = (torch.sigmoid(_rand((n, heads), i)).to(torch.bfloat16).to(device)
+                   for i, n in ((75, rows), (76, text_rows)))
+    alpha = torch.rand(frames, heads, dim, generator=torch.Generator().manual_seed(77)).to(device)
+    flags = dict(k_features=k_features, v_features=v_features, a_fp32=a_fp32)
+    video, text = branch.frame_statistics_with_text(k, v, beta, frames, tokens, tk, tv, tbeta, **flags)
+    want = branch.frame_statistics_raw(k, v, beta, frames, tokens, **flags)
+    want_text = branch.frame_statistics_raw(tk, tv, tbeta, 1, text_rows, a_fp32=a_fp32)
+    for got, ref in zip((*video, *text), (*want, *want_text)):
+        assert torch.equal(got, ref)
+    rule = branch.VdnDelta()
+    with branch.cholesky_runtime_scope() as checks:
+        phi, jay, text_jay = rule.factor_apply_with_text(alpha, *want, *want_text)
+        assert [tuple(s.shape) for s in checks.statuses] == [(1, heads), (frames, heads)]
+        ref = rule.factor_apply(alpha, *want)
+        ref_text = rule.factor_apply(None, *want_text, jay_scale=branch.TEXT_STATE_SCALE, need_phi=False)
+    for got, w in ((phi, ref[0]), (jay, ref[1]), (text_jay, ref_text[1])):
+        assert torch.equal(got, w)
+
+
 @pytest.mark.parametrize("text,bridge", [(False, "alpha"), (True, "alpha"), (True, "none")])
 def test_readout_epilogue(device, text, bridge):
     from vdn_h3_amd import branch
