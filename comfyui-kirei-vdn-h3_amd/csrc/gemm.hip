@@ -75,13 +75,8 @@ extern "C" int vdnh3_gemm(int kind, const void *A, int64_t lda, const void *B, i
                    "gemm: a_scale must have 1 or M entries");
   VDNH3_HOST_CHECK(!b_scale || b_scale_n == 1 || b_scale_n == N, VDNH3_ERR_INVALID,
                    "gemm: b_scale must have 1 or N entries");
-  const int esize = out_type == kOutBF16 ? 2 : 4;
-  const uintptr_t c_addr = reinterpret_cast<uintptr_t>(C);
-  const int vec = N % 8 == 0 && ldc % 8 == 0 && c_addr % 16 == 0             ? 8
-                  : N % 4 == 0 && ldc % 4 == 0 && c_addr % (4 * esize) == 0 ? 4
-                                                                            : 1;
   GemmEpi epi{a_scale, b_scale, b_scale_n, a_scale_n, alpha, bias, bias_bf16, act & 1, act >> 1, out_type, accumulate,
-              round_linear, vec};
+              round_linear};
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (kind) {
     case kBF16:

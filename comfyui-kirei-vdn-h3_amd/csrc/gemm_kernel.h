@@ -51,7 +51,6 @@ struct GemmEpi {
   int out_type;       // OutType
   int accumulate;     // C += epi(acc)
   int round_linear;   // bf16 output: round the linear result to bf16 before the activation
-  int vec;            // elements of C a lane may store at once: 8, 4 or 1 (N, ldc and C allow it)
 };
 
 struct GemmArgs {
@@ -94,6 +93,11 @@ template <typename V, typename P>
 __device__ __forceinline__ V stream_load(const P *p) {
   return __builtin_nontemporal_load(reinterpret_cast<const V *>(p));
 }
+// 16 bytes of C at the alignment of its elements (any N and ldc; global accesses of any alignment are one
+// instruction here)
+typedef u32x4_t __attribute__((aligned(2))) u32x4_a2_t;
+typedef u32x4_t __attribute__((aligned(4))) u32x4_a4_t;
+typedef f32x4_t __attribute__((aligned(4))) f32x4_a4_t;
 
 // Epilogue operands. Loaded at the start of the kernel, one column (its scale times alpha, its bias) and
 // MI / 4 rows per lane, so that their latency hides behind the main loop at 2 + MI / 4 registers; the
@@ -123,15 +127,15 @@ __device__ __forceinline__ EpiOperands<MI> load_epi_operands(const GemmEpi &epi,
 }
 
 // Lane (l16 = lane % 16, g = lane / 16) holds, of row 16 i + l16 of the wavefront's block, columns
-// 32 jp + 8 g + 0 .. 7 in acc[i][2 jp] and acc[i][2 jp + 1]. bf16 output with 16-byte alignment: lanes of
-// an even and the next odd row swap halves (one DPP move per word), so that one store instruction writes
-// eight whole 128-byte rows of the block; with 64-byte pieces of 16 rows instead the GEMM took 3-5% longer.
+// 32 jp + 8 g + 0 .. 7 in acc[i][2 jp] and acc[i][2 jp + 1]. bf16 output: lanes of an even and the next odd
+// row swap halves (one DPP move per word), so that one store instruction writes eight whole 128-byte rows of
+// the block; with 64-byte pieces of 16 rows instead the GEMM took 3-5% longer. A lane whose eight columns
+// reach past N stores them one by one; nothing else depends on N or the alignment of C's rows.
 template <int OUT, bool ACT, bool ACCUM, int MI, typename Acc>
 __device__ __forceinline__ void store_block(const Acc (&acc)[MI][4], float *stage, const EpiOperands<MI> &eo,
                                             const GemmEpi &epi, void *C, int64_t ldc, int M, int N, int mb, int nb,
                                             int lane) {
   const int l16 = lane & 15, g = lane >> 4;
-  const int vec = epi.vec;
   float cs[16], bs[16];
   if constexpr (OUT != kOutI32) {
 #pragma unroll
@@ -163,115 +167,98 @@ __device__ __forceinline__ void store_block(const Acc (&acc)[MI][4], float *stag
     }
   };
   if constexpr (OUT == kOutBF16) {
-    if (vec == 8) {
-      const bool odd = lane & 1;
-      const int n = nb + 8 * g + (odd ? 32 : 0);
-      const int m0 = mb + (l16 & ~1);
-      uint16_t *cp = static_cast<uint16_t *>(C) + (int64_t)m0 * ldc + n;
-      // when accumulating, the old values of four block rows are loaded together, before their stores
-      constexpr int kBatch = ACCUM ? 4 : 1;
+    const bool odd = lane & 1;
+    const int n = nb + 8 * g + (odd ? 32 : 0);
+    const int m0 = mb + (l16 & ~1);
+    uint16_t *cp = static_cast<uint16_t *>(C) + (int64_t)m0 * ldc + n;
+    // when accumulating, the old values of four block rows are loaded together, before their stores
+    constexpr int kBatch = ACCUM ? 4 : 1;
 #pragma unroll
-      for (int i0 = 0; i0 < MI; i0 += kBatch) {
-        u32x4_t old[kBatch][2];
-        if constexpr (ACCUM) {
+    for (int i0 = 0; i0 < MI; i0 += kBatch) {
+      u32x4_t old[kBatch][2];
+      if constexpr (ACCUM) {
 #pragma unroll
-          for (int b = 0; b < kBatch; ++b)
+        for (int b = 0; b < kBatch; ++b)
 #pragma unroll
-            for (int r = 0; r < 2; ++r)
-              if (i0 + b < MI && n < N && m0 + 16 * (i0 + b) + r < M)
-                old[b][r] = stream_load<u32x4_t>(cp + (int64_t)(16 * (i0 + b) + r) * ldc);
+          for (int r = 0; r < 2; ++r)
+            if (i0 + b < MI && n + 8 <= N && m0 + 16 * (i0 + b) + r < M)
+              old[b][r] = stream_load<u32x4_a2_t>(cp + (int64_t)(16 * (i0 + b) + r) * ldc);
+      }
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const int i = i0 + b;
+        if (i >= MI) break;
+        u32x4_t w[2], o[2];
+#pragma unroll
+        for (int jp = 0; jp < 2; ++jp) {
+          float v[8];
+          values(i, jp, v);
+#pragma unroll
+          for (int h = 0; h < 4; ++h) w[jp][h] = pack_bf2(v[2 * h], v[2 * h + 1]);
         }
 #pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-          const int i = i0 + b;
-          if (i >= MI) break;
-          u32x4_t w[2], o[2];
+        for (int h = 0; h < 4; ++h) {
+          const uint32_t x = odd ? w[0][h] : w[1][h];
+          const uint32_t y = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+          o[0][h] = odd ? y : w[0][h];
+          o[1][h] = odd ? w[1][h] : y;
+        }
 #pragma unroll
-          for (int jp = 0; jp < 2; ++jp) {
-            float v[8];
-            values(i, jp, v);
-#pragma unroll
-            for (int h = 0; h < 4; ++h) w[jp][h] = pack_bf2(v[2 * h], v[2 * h + 1]);
-          }
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            const uint32_t x = odd ? w[0][h] : w[1][h];
-            const uint32_t y = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true);  // lane ^ 1
-            o[0][h] = odd ? y : w[0][h];
-            o[1][h] = odd ? w[1][h] : y;
-          }
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
+        for (int r = 0; r < 2; ++r) {
+          uint16_t *row = cp + (int64_t)(16 * i + r) * ldc;
+          if (m0 + 16 * i + r >= M) continue;
+          if (n + 8 <= N) {
             if constexpr (ACCUM) {
 #pragma unroll
               for (int h = 0; h < 4; ++h)
                 o[r][h] = pack_bf2(bf2f(old[b][r][h] & 0xffff) + bf2f(o[r][h] & 0xffff),
                                    bf2f(old[b][r][h] >> 16) + bf2f(o[r][h] >> 16));
             }
-            if (n < N && m0 + 16 * i + r < M) stream_store(o[r], cp + (int64_t)(16 * i + r) * ldc);
+            stream_store<u32x4_a2_t>(o[r], row);
+          } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const uint16_t e = (uint16_t)(o[r][k >> 1] >> (16 * (k & 1)));
+              if (n + k < N) row[k] = ACCUM ? f2bf(bf2f(row[k]) + bf2f(e)) : e;
+            }
           }
         }
       }
-      return;
     }
-  }
+  } else {
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = mb + 16 * i + l16;
+    for (int i = 0; i < MI; ++i) {
+      const int m = mb + 16 * i + l16;
 #pragma unroll
-    for (int jp = 0; jp < 2; ++jp) {
-      const int n = nb + 32 * jp + 8 * g;
-      if (m >= M || n >= N) continue;
-      const int64_t off = (int64_t)m * ldc + n;
-      if constexpr (OUT == kOutI32) {
-        int32_t *cp = static_cast<int32_t *>(C) + off;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (vec >= 4) {
-            if (n + 4 * h < N) stream_store(__builtin_bit_cast(u32x4_t, acc[i][2 * jp + h]), cp + 4 * h);
-          } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const auto e = acc[i][2 * jp + h][k];
-              if (n + 4 * h + k < N) cp[4 * h + k] = (int32_t)e;
-            }
-          }
-        }
-      } else {
+      for (int jp = 0; jp < 2; ++jp) {
+        if (m >= M) continue;
         float v[8];
-        values(i, jp, v);
+        if constexpr (OUT == kOutF32) values(i, jp, v);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          if (n + 4 * h >= N) continue;
-          const float *vh = v + 4 * h;
-          if constexpr (OUT == kOutF32) {
-            float *cp = static_cast<float *>(C) + off + 4 * h;
-            if (vec >= 4) {
-              f32x4_t o = {vh[0], vh[1], vh[2], vh[3]};
-              if constexpr (ACCUM) o += stream_load<f32x4_t>(cp);
-              stream_store(o, cp);
+          const int n = nb + 32 * jp + 8 * g + 4 * h;
+          const int64_t off = (int64_t)m * ldc + n;
+          if constexpr (OUT == kOutI32) {
+            int32_t *cp = static_cast<int32_t *>(C) + off;
+            if (n + 4 <= N) {
+              stream_store<u32x4_a4_t>(__builtin_bit_cast(u32x4_t, acc[i][2 * jp + h]), cp);
             } else {
 #pragma unroll
-              for (int k = 0; k < 4; ++k)
-                if (n + 4 * h + k < N) cp[k] = ACCUM ? cp[k] + vh[k] : vh[k];
+              for (int k = 0; k < 4; ++k) {
+                const auto e = acc[i][2 * jp + h][k];
+                if (n + k < N) cp[k] = (int32_t)e;
+              }
             }
           } else {
-            uint16_t *cp = static_cast<uint16_t *>(C) + off + 4 * h;
-            if (vec >= 4) {
-              uint32_t lo, hi;
-              if constexpr (ACCUM) {
-                const u32x2_t o = stream_load<u32x2_t>(cp);
-                lo = pack_bf2(bf2f(o.x & 0xffff) + round_bf(vh[0]), bf2f(o.x >> 16) + round_bf(vh[1]));
-                hi = pack_bf2(bf2f(o.y & 0xffff) + round_bf(vh[2]), bf2f(o.y >> 16) + round_bf(vh[3]));
-              } else {
-                lo = pack_bf2(vh[0], vh[1]);
-                hi = pack_bf2(vh[2], vh[3]);
-              }
-              stream_store(u32x2_t{lo, hi}, cp);
+            float *cp = static_cast<float *>(C) + off;
+            if (n + 4 <= N) {
+              f32x4_t o = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+              if constexpr (ACCUM) o += stream_load<f32x4_a4_t>(cp);
+              stream_store<f32x4_a4_t>(o, cp);
             } else {
 #pragma unroll
               for (int k = 0; k < 4; ++k)
-                if (n + 4 * h + k < N) cp[k] = f2bf(ACCUM ? bf2f(cp[k]) + round_bf(vh[k]) : vh[k]);
+                if (n + k < N) cp[k] = ACCUM ? cp[k] + v[4 * h + k] : v[4 * h + k];
             }
           }
         }
