@@ -342,6 +342,63 @@ __device__ __forceinline__ void store_rows(const f32x4_t (&oacc)[D / 16][kNQ], c
   }
 }
 
+// The partial result of a wavefront's rows over one split of their key tiles: O^T unnormalised, the running
+// max (base 2) and the row sum, [split][head][row][D] and [split][head][row][2] fp32.
+struct Partial {
+  float *o, *ml;  // null: the whole key set in one workgroup
+};
+template <int D>
+__device__ __forceinline__ void store_partial(const f32x4_t (&oacc)[D / 16][kNQ], const f32x4_t (&l)[kNQ],
+                                              const float (&m_run)[kNQ], int q0, int q1, const Partial &part,
+                                              int64_t head_rows, int l16, int g) {
+#pragma unroll
+  for (int n = 0; n < kNQ; ++n) {
+    const int qr = q0 + 16 * n + l16;
+    if (qr >= q1) continue;
+    float *op = part.o + (head_rows + qr) * D + 4 * g;
+#pragma unroll
+    for (int m = 0; m < D / 16; ++m) *reinterpret_cast<f32x4_t *>(op + 16 * m) = oacc[m][n];
+    if (g == 0) *reinterpret_cast<float2 *>(part.ml + (head_rows + qr) * 2) = make_float2(m_run[n], l[n][0]);
+  }
+}
+
+// Combines the splits of every row: O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, m = max m_s; the
+// rounding and the gate as store_rows. One thread per 8 channels of a (row, head).
+template <int D>
+__global__ __launch_bounds__(256) void combine_kernel(Partial part, int splits, int seq, int heads,
+                                                      const uint16_t *__restrict__ gate, int64_t g_row,
+                                                      uint16_t *__restrict__ out, int64_t o_row, int64_t o_head) {
+  constexpr int CH = D / 8;
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t rows = (int64_t)heads * seq;
+  if (e >= rows * CH) return;
+  const int64_t hr = e / CH;
+  const int c = (int)(e - hr * CH), head = (int)(hr / seq), row = (int)(hr - (int64_t)head * seq);
+  float m = -INFINITY;
+  for (int s = 0; s < splits; ++s) m = fmaxf(m, part.ml[(s * rows + hr) * 2]);
+  f32x4_t o[2] = {};
+  float l = 0.f;
+  for (int s = 0; s < splits; ++s) {
+    const float2 ml = *reinterpret_cast<const float2 *>(part.ml + (s * rows + hr) * 2);
+    const float w = __builtin_amdgcn_exp2f(ml.x - m);
+    const f32x4_t *op = reinterpret_cast<const f32x4_t *>(part.o + (s * rows + hr) * D + 8 * c);
+    o[0] += w * op[0];
+    o[1] += w * op[1];
+    l += w * ml.y;
+  }
+  const float inv = 1.f / l;
+  const float gv = gate ? bf2f(gate[(int64_t)row * g_row + head]) : 1.f;
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    v[j] = round_bf(o[j >> 2][j & 3] * inv);
+    if (gate) v[j] *= gv;
+  }
+  uint16_t *dst = out + (int64_t)row * o_row + (int64_t)head * o_head + 8 * c;  // 8-byte aligned
+  *reinterpret_cast<uint2 *>(dst) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+  *reinterpret_cast<uint2 *>(dst + 4) = make_uint2(pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7]));
+}
+
 // ---------------------------------------------------------------------------------
 // Two-group ping-pong over the key tiles t = 0..T-1 of a work item (256 query rows of one head).
 // Waves 0-3 (group A) and 4-7 (group B) each own 32 query rows; wave w and w + 4 share a SIMD.
@@ -366,7 +423,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
     int64_t k_head, const uint16_t *__restrict__ vt, int s_pad, uint16_t *__restrict__ out, int64_t o_row,
     int64_t o_head, const uint16_t *__restrict__ gate, int64_t g_row, int seq, float scale_log2,
     const int4 *__restrict__ items, int n_items, const int2 *__restrict__ tiles, int per_xcd, int total,
-    const uint16_t *__restrict__ q_weight, float q_eps) {
+    const uint16_t *__restrict__ q_weight, float q_eps, Partial part) {
   constexpr int KC = D / 8;    // 16-byte chunks per K row
   constexpr int NS = D / 32;   // k-steps of the QK^T contraction
   constexpr int NO = D / 16;   // 16-row blocks of O^T
@@ -384,7 +441,9 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   if (L >= total) return;
   const int head = L / n_items;
   const int4 item = items[L - head * n_items];
-  const int q0 = item.x, q1 = item.y, toff = item.z, T = item.w;
+  // grid.y splits of the item's key tiles (the host keeps it at or below every item's tile count)
+  const int t0 = item.w * (int)blockIdx.y / (int)gridDim.y, t1 = item.w * ((int)blockIdx.y + 1) / (int)gridDim.y;
+  const int q0 = item.x, q1 = item.y, toff = item.z + t0, T = t1 - t0;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int l16 = lane & 15, g = lane >> 4;
@@ -622,7 +681,11 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   }
 
   wait_vm_lds<0>();  // no tile load may land in LDS after the workgroup ends
-  store_rows<D>(oacc, l_run, q0 + wave * 32, q1, gate, g_row, head, out, o_row, o_head, l16, g);
+  if (part.o)
+    store_partial<D>(oacc, l_run, m_run, q0 + wave * 32, q1, part,
+                     ((int64_t)blockIdx.y * (total / n_items) + head) * seq, l16, g);
+  else
+    store_rows<D>(oacc, l_run, q0 + wave * 32, q1, gate, g_row, head, out, o_row, o_head, l16, g);
 }
 
 template <int D>
@@ -639,15 +702,23 @@ template <int D, bool QNORM>
 int launch_attn(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *k, int64_t k_row, int64_t k_head,
                 uint16_t *out, int64_t o_row, int64_t o_head, const uint16_t *gate, int64_t gate_row, int seq,
                 int heads, float scale, const int32_t *items, int32_t n_items, const int32_t *tiles,
-                const void *workspace, hipStream_t stream, const uint16_t *q_weight = nullptr, float q_eps = 0.f) {
+                const void *workspace, hipStream_t stream, const uint16_t *q_weight = nullptr, float q_eps = 0.f,
+                int splits = 1, float *partial = nullptr) {
   const int s_pad = pad_rows(seq);
   const int total = n_items * heads;
   const int per_xcd = (total + 7) / 8;
-  hipLaunchKernelGGL((window_attn_kernel<D, QNORM>), dim3(per_xcd * 8), dim3(kThreads), 0, stream, q, q_row, q_head, k,
+  Partial part{nullptr, nullptr};
+  if (splits > 1) part = Partial{partial, partial + (size_t)splits * heads * seq * D};
+  hipLaunchKernelGGL((window_attn_kernel<D, QNORM>), dim3(per_xcd * 8, splits), dim3(kThreads), 0, stream, q, q_row, q_head, k,
                      k_row, k_head, static_cast<const uint16_t *>(workspace), s_pad, out, o_row, o_head, gate,
                      gate_row, seq, scale * 1.4426950408889634f, reinterpret_cast<const int4 *>(items), n_items,
-                     reinterpret_cast<const int2 *>(tiles), per_xcd, total, q_weight, q_eps);
-  return check_launch("window_attn");
+                     reinterpret_cast<const int2 *>(tiles), per_xcd, total, q_weight, q_eps, part);
+  int rc = check_launch("window_attn");
+  if (rc || splits <= 1) return rc;
+  const int64_t threads = (int64_t)heads * seq * (D / 8);
+  hipLaunchKernelGGL(combine_kernel<D>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, part, splits, seq,
+                     heads, gate, gate_row, out, o_row, o_head);
+  return check_launch("window_attn combine");
 }
 
 template <int D>
@@ -720,25 +791,65 @@ extern "C" int vdnh3_window_vt_prepass(const uint16_t *v, int64_t v_row, int64_t
                          : vdnh3::launch_prepass<64>(v, v_row, v_head, seq, heads, workspace, s);
 }
 
+extern "C" size_t vdnh3_window_partial_bytes(int seq, int heads, int head_dim, int splits) {
+  if (seq <= 0 || heads <= 0 || head_dim <= 0 || splits <= 1) return 0;
+  return size_t(splits) * size_t(heads) * size_t(seq) * size_t(head_dim + 2) * sizeof(float);
+}
+
+namespace vdnh3 {
+namespace {
+
+int check_attn(const uint16_t *out, int64_t o_row, int64_t o_head, const int32_t *items, const int32_t *tiles,
+               int32_t n_items) {
+  VDNH3_HOST_CHECK(out != nullptr && o_row % 4 == 0 && o_head % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0,
+                   VDNH3_ERR_INVALID, "out must be 8-byte aligned with strides that are multiples of 4 elements");
+  VDNH3_HOST_CHECK(items != nullptr && tiles != nullptr && n_items > 0, VDNH3_ERR_INVALID, "empty window plan");
+  return VDNH3_OK;
+}
+
+int check_partial(int seq, int heads, int head_dim, int splits, const float *partial, size_t partial_bytes) {
+  VDNH3_HOST_CHECK(splits >= 1 && splits <= 64, VDNH3_ERR_INVALID, "splits must be 1 to 64, got %d", splits);
+  VDNH3_HOST_CHECK(splits == 1 || (partial && reinterpret_cast<uintptr_t>(partial) % 16 == 0 &&
+                                   partial_bytes >= vdnh3_window_partial_bytes(seq, heads, head_dim, splits)),
+                   VDNH3_ERR_INVALID, "the partial buffer must be 16-byte aligned and hold %zu bytes, got %zu",
+                   vdnh3_window_partial_bytes(seq, heads, head_dim, splits), partial_bytes);
+  return VDNH3_OK;
+}
+
+}  // namespace
+}  // namespace vdnh3
+
+extern "C" int vdnh3_window_attn_prepared_split(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *k,
+                                                int64_t k_row, int64_t k_head, uint16_t *out, int64_t o_row,
+                                                int64_t o_head, const uint16_t *gate, int64_t gate_row, int seq,
+                                                int heads, int head_dim, float scale, const int32_t *items,
+                                                int32_t n_items, const int32_t *tiles, const void *workspace,
+                                                size_t workspace_bytes, int splits, float *partial,
+                                                size_t partial_bytes, void *stream) {
+  int rc = vdnh3::check_common(seq, heads, head_dim, workspace, workspace_bytes);
+  if (!rc) rc = vdnh3::check_vec(q, q_row, q_head, "q");
+  if (!rc) rc = vdnh3::check_vec(k, k_row, k_head, "k");
+  if (!rc) rc = vdnh3::check_attn(out, o_row, o_head, items, tiles, n_items);
+  if (!rc) rc = vdnh3::check_partial(seq, heads, head_dim, splits, partial, partial_bytes);
+  if (rc) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (head_dim == 128)
+    return vdnh3::launch_attn<128, false>(q, q_row, q_head, k, k_row, k_head, out, o_row, o_head, gate, gate_row, seq,
+                                          heads, scale, items, n_items, tiles, workspace, s, nullptr, 0.f, splits,
+                                          partial);
+  return vdnh3::launch_attn<64, false>(q, q_row, q_head, k, k_row, k_head, out, o_row, o_head, gate, gate_row, seq,
+                                       heads, scale, items, n_items, tiles, workspace, s, nullptr, 0.f, splits, partial);
+}
+
 extern "C" int vdnh3_window_attn_prepared(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *k,
                                           int64_t k_row, int64_t k_head, uint16_t *out, int64_t o_row,
                                           int64_t o_head, const uint16_t *gate, int64_t gate_row, int seq, int heads,
                                           int head_dim, float scale, const int32_t *items, int32_t n_items,
                                           const int32_t *tiles, const void *workspace, size_t workspace_bytes,
                                           void *stream) {
-  int rc = vdnh3::check_common(seq, heads, head_dim, workspace, workspace_bytes);
-  if (!rc) rc = vdnh3::check_vec(q, q_row, q_head, "q");
-  if (!rc) rc = vdnh3::check_vec(k, k_row, k_head, "k");
-  if (rc) return rc;
-  VDNH3_HOST_CHECK(out != nullptr && o_row % 4 == 0 && o_head % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0,
-                   VDNH3_ERR_INVALID, "out must be 8-byte aligned with strides that are multiples of 4 elements");
-  VDNH3_HOST_CHECK(items != nullptr && tiles != nullptr && n_items > 0, VDNH3_ERR_INVALID, "empty window plan");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (head_dim == 128)
-    return vdnh3::launch_attn<128, false>(q, q_row, q_head, k, k_row, k_head, out, o_row, o_head, gate, gate_row, seq,
-                                      heads, scale, items, n_items, tiles, workspace, s);
-  return vdnh3::launch_attn<64, false>(q, q_row, q_head, k, k_row, k_head, out, o_row, o_head, gate, gate_row, seq, heads,
-                                   scale, items, n_items, tiles, workspace, s);
+  return vdnh3_window_attn_prepared_split(q, q_row, q_head, k, k_row, k_head, out, o_row, o_head, gate, gate_row, seq,
+                                          heads, head_dim, scale, items, n_items, tiles, workspace, workspace_bytes, 1,
+                                          nullptr, 0, stream);
 }
 
 extern "C" int vdnh3_window_attn_fwd(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *k,
@@ -785,11 +896,12 @@ extern "C" int vdnh3_window_qkv_prepass(const uint16_t *q, int64_t q_row, int64_
                                                          seq, heads, workspace, s);
 }
 
-extern "C" int vdnh3_window_attn_qnorm(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *q_weight,
+extern "C" int vdnh3_window_attn_qnorm_split(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *q_weight,
                                        float q_eps, uint16_t *out, int64_t o_row, int64_t o_head, const uint16_t *gate,
                                        int64_t gate_row, int seq, int heads, int head_dim, float scale,
                                        const int32_t *items, int32_t n_items, const int32_t *tiles,
-                                       const void *workspace, size_t workspace_bytes, void *stream) {
+                                       const void *workspace, size_t workspace_bytes, int splits, float *partial,
+                                       size_t partial_bytes, void *stream) {
   int rc = vdnh3::check_common(seq, heads, head_dim, workspace, workspace_bytes);
   if (!rc) rc = vdnh3::check_vec(q, q_row, q_head, "q");
   if (!rc) rc = vdnh3::check_vec(q_weight, 0, 0, "q_weight");
@@ -797,9 +909,9 @@ extern "C" int vdnh3_window_attn_qnorm(const uint16_t *q, int64_t q_row, int64_t
   VDNH3_HOST_CHECK(workspace_bytes >= vdnh3_window_norm_workspace_bytes(seq, heads, head_dim, 0), VDNH3_ERR_INVALID,
                    "workspace of %zu bytes is smaller than the %zu the normalising attention reads", workspace_bytes,
                    vdnh3_window_norm_workspace_bytes(seq, heads, head_dim, 0));
-  VDNH3_HOST_CHECK(out != nullptr && o_row % 4 == 0 && o_head % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0,
-                   VDNH3_ERR_INVALID, "out must be 8-byte aligned with strides that are multiples of 4 elements");
-  VDNH3_HOST_CHECK(items != nullptr && tiles != nullptr && n_items > 0, VDNH3_ERR_INVALID, "empty window plan");
+  rc = vdnh3::check_attn(out, o_row, o_head, items, tiles, n_items);
+  if (!rc) rc = vdnh3::check_partial(seq, heads, head_dim, splits, partial, partial_bytes);
+  if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int s_pad = vdnh3::pad_rows(seq);
   // the normalised keys follow the V^T copy in the workspace: [heads][s_pad][head_dim]
@@ -807,7 +919,19 @@ extern "C" int vdnh3_window_attn_qnorm(const uint16_t *q, int64_t q_row, int64_t
   const int64_t kn_row = head_dim, kn_head = (int64_t)s_pad * head_dim;
   if (head_dim == 128)
     return vdnh3::launch_attn<128, true>(q, q_row, q_head, kn, kn_row, kn_head, out, o_row, o_head, gate, gate_row,
-                                         seq, heads, scale, items, n_items, tiles, workspace, s, q_weight, q_eps);
+                                         seq, heads, scale, items, n_items, tiles, workspace, s, q_weight, q_eps, splits,
+                                         partial);
   return vdnh3::launch_attn<64, true>(q, q_row, q_head, kn, kn_row, kn_head, out, o_row, o_head, gate, gate_row, seq,
-                                      heads, scale, items, n_items, tiles, workspace, s, q_weight, q_eps);
+                                      heads, scale, items, n_items, tiles, workspace, s, q_weight, q_eps, splits,
+                                         partial);
+}
+
+extern "C" int vdnh3_window_attn_qnorm(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *q_weight,
+                                       float q_eps, uint16_t *out, int64_t o_row, int64_t o_head, const uint16_t *gate,
+                                       int64_t gate_row, int seq, int heads, int head_dim, float scale,
+                                       const int32_t *items, int32_t n_items, const int32_t *tiles,
+                                       const void *workspace, size_t workspace_bytes, void *stream) {
+  return vdnh3_window_attn_qnorm_split(q, q_row, q_head, q_weight, q_eps, out, o_row, o_head, gate, gate_row, seq, heads,
+                                       head_dim, scale, items, n_items, tiles, workspace, workspace_bytes, 1, nullptr,
+                                       0, stream);
 }

@@ -142,7 +142,71 @@ Plan make_plan(const Geometry &g, int block_m, int block_n) {
   return p;
 }
 
+// How a call with `heads` heads is best divided: the most query rows of an item (256, 128 or 64) and how many
+// workgroups share an item's key tiles, by the least estimated time. A workgroup takes its tiles plus about five
+// (prologue, first loads, epilogue), one workgroup per CU; more than 256 of them share the CUs evenly with
+// half the longest left over. us per tile and workgroup, measured at 4, 9 and 70 tiles: 1.95 / 1.68 / 1.62 with 256
+// / 128 / 64 rows at head dim 128, 1.50 / 1.23 / 1.17 at 64 (below 129 rows one of the workgroup's two groups is
+// idle and the other's phases have the SIMDs to themselves). Splits cost a combining launch (12 us with its host
+// side) and their fp32 partials written and read (about 6 TB/s). Whole items of 256 rows stay unless 5% are gained,
+// so a call that fills the GPU is left as it is. Measured, whole items of 256 rows against the choice: one head of
+// 6,700 rows 151 -> 43 us (8 splits), one head of 40,688 rows 850 -> 630 us, four heads of 6,700 rows 158 -> 98 us,
+// two heads of 848 rows of 64 (64 rows an item, whole) 21 -> 16 us.
+struct Shape {
+  int block_m, splits;
+};
+
+Shape shape_call(const std::vector<Run> &runs, int block_n, int64_t heads, int seq, int dim) {
+  struct Count {
+    int64_t rows, tiles;
+  };
+  std::vector<Count> counts;
+  int64_t fewest = INT64_MAX, most = 0;
+  for (const Run &r : runs) {
+    std::vector<int32_t> tiles;
+    tiles_of(r.keys, block_n, &tiles);
+    const int64_t n = int64_t(tiles.size() / 2);
+    counts.push_back({r.q1 - r.q0, n});
+    fewest = std::min(fewest, n);
+    most = std::max(most, n);
+  }
+  Shape best{256, 1};
+  double best_us = -1;
+  for (const int bm : {256, 128, 64}) {
+    int64_t items = 0, work = 0;
+    for (const Count &c : counts) {
+      const int64_t n = (c.rows + bm - 1) / bm;
+      items += n;
+      work += n * c.tiles;
+    }
+    const double tile_us = dim > 64 ? (bm == 256 ? 1.95 : bm == 128 ? 1.68 : 1.62) : (bm == 256 ? 1.50 : bm == 128 ? 1.23 : 1.17);
+    for (int s = 1; s <= std::min<int64_t>(fewest, 16); ++s) {
+      const double longest = double(most) / s + 5;
+      double us = items * heads * s <= 256 ? longest : double(work + 5 * s * items) * heads / 256 + longest / 2;
+      us *= tile_us;
+      if (s > 1) us += 12 + 8e-6 * s * heads * seq * dim / 6;
+      if (best_us < 0) best_us = 0.95 * us;  // whole items of 256 rows
+      else if (us < best_us) best = {bm, s}, best_us = us;
+    }
+  }
+  return best;
+}
+
 }  // namespace
+
+extern "C" int vdnh3_window_plan_shape(int seq, int video_start, int video_end, int num_frames, int tokens_per_frame,
+                                       const int32_t *bounds, int anchor_mode, int block_n, int heads, int head_dim,
+                                       int32_t *block_m, int32_t *splits) {
+  Geometry g{seq, video_start, video_end, num_frames, tokens_per_frame, anchor_mode, bounds};
+  int rc = validate(g, 256, block_n);
+  if (rc) return rc;
+  Shape shape{256, 1};
+  const std::vector<Run> runs = runs_of(g);
+  if (heads > 0 && head_dim > 0 && !runs.empty()) shape = shape_call(runs, block_n, heads, seq, head_dim);
+  if (block_m) *block_m = shape.block_m;
+  if (splits) *splits = shape.splits;
+  return VDNH3_OK;
+}
 
 extern "C" int vdnh3_window_plan_size(int seq, int video_start, int video_end, int num_frames,
                                       int tokens_per_frame, const int32_t *bounds, int anchor_mode,

@@ -32,10 +32,13 @@ SIGNATURES = {
     "vdnh3_abi_version": (_c_int, []),
     "vdnh3_window_plan_size": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _p_i32, _c_int, _c_int, _c_int,
                                         _p_i32, _p_i32, _p_i64]),
+    "vdnh3_window_plan_shape": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _p_i32, _c_int, _c_int, _c_int,
+                                         _c_int, _p_i32, _p_i32]),
     "vdnh3_window_plan_build": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _p_i32, _c_int, _c_int, _c_int,
                                          _p_i32, _c_i32, _p_i32, _c_i32]),
     "vdnh3_window_block_m": (_c_int, []),
     "vdnh3_window_block_n": (_c_int, []),
+    "vdnh3_window_partial_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "vdnh3_window_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),
     "vdnh3_window_attn_fwd": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64,
                                        _vp, _c_i64, _c_i64, _vp, _c_i64,
@@ -45,12 +48,19 @@ SIGNATURES = {
     "vdnh3_window_attn_prepared": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64,
                                             _vp, _c_i64, _c_int, _c_int, _c_int, _c_float,
                                             _vp, _c_i32, _vp, _vp, _c_size, _vp]),
+    "vdnh3_window_attn_prepared_split": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64,
+                                            _vp, _c_i64, _c_int, _c_int, _c_int, _c_float,
+                                            _vp, _c_i32, _vp, _vp, _c_size, _c_int, _vp,
+                                          _c_size, _vp]),
     "vdnh3_window_norm_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "vdnh3_window_qkv_prepass": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_float, _vp, _c_i64, _c_i64, _vp, _c_float,
                                           _vp, _c_i64, _c_i64, _vp, _c_i64, _c_int, _c_int, _c_int, _c_int,
                                           _vp, _c_size, _vp]),
     "vdnh3_window_attn_qnorm": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_float, _vp, _c_i64, _c_i64, _vp, _c_i64,
                                          _c_int, _c_int, _c_int, _c_float, _vp, _c_i32, _vp, _vp, _c_size, _vp]),
+    "vdnh3_window_attn_qnorm_split": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_float, _vp, _c_i64, _c_i64, _vp, _c_i64,
+                                         _c_int, _c_int, _c_int, _c_float, _vp, _c_i32, _vp, _vp, _c_size, _c_int, _vp,
+                                          _c_size, _vp]),
     "vdnh3_gemm": (_c_int, [_c_int, _vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_int, _c_int, _c_int,
                             _vp, _c_int, _vp, _c_int, _c_float, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "vdnh3_quant_rows": (_c_int, [_c_int, _vp, _c_i64, _c_int, _c_int, _vp, _c_i64, _vp, _vp]),

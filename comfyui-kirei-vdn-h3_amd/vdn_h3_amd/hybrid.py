@@ -306,11 +306,12 @@ class _VDNBlockForward:
         cache = self.state.window_cache
         if layout.full_cover:
             self.state.last_attention_backend = "dense_exact"
-            return cache.plan(layout.seq_len, 0, layout.seq_len, 1, layout.seq_len, [(0, 0)], "none", device)
+            return cache.plan(layout.seq_len, 0, layout.seq_len, 1, layout.seq_len, [(0, 0)], "none", device,
+                              self.heads, self.head_dim)
         self.state.last_attention_backend = _window.resolve_attention_backend(self.state.attention_backend,
                                                                               cache=cache)
         return cache.plan(layout.seq_len, layout.video_start, layout.video_end, layout.num_frames,
-                          layout.tokens_per_frame, layout.bounds, layout.anchor_frames, device)
+                          layout.tokens_per_frame, layout.bounds, layout.anchor_frames, device, self.heads, self.head_dim)
 
     def _forward(self, x, layout, rope_freqs):
         state, attn, heads, head_dim = self.state, self.attn, self.heads, self.head_dim

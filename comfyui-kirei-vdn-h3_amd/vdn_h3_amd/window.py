@@ -86,10 +86,30 @@ class WindowPlan:
     n_items: int
     n_tiles: int
     pairs_per_head: int     # allowed (query, key) pairs per head
+    block_m: int = 256      # most query rows of an item
+    splits: int = 1         # workgroups that divide an item's key tiles (at most its fewest tiles)
 
 
-def build_plan_host(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames):
-    """Run the C++ planner on the host; returns ``(items[n,4], tiles[m,2], pairs)`` CPU int32 tensors."""
+def build_plan_host(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, block_m=None):
+    """Run the C++ planner on the host; returns ``(items[n,4], tiles[m,2], pairs)`` CPU int32 tensors.
+    ``block_m``: most query rows of an item (default and at most the kernel's block, ``vdnh3_window_block_m``)."""
+    lib = _lib.lib()
+    geometry = _plan_geometry(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames)
+    bm, bn = block_m or lib.vdnh3_window_block_m(), lib.vdnh3_window_block_n()
+    n_items, n_tiles, pairs = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
+    _lib.check(lib.vdnh3_window_plan_size(*geometry, bm, bn, ctypes.byref(n_items), ctypes.byref(n_tiles),
+                                          ctypes.byref(pairs)), "window plan")
+    # one buffer for both, so that a device copy of the plan is one transfer
+    words = torch.empty(4 * n_items.value + 2 * n_tiles.value, dtype=torch.int32)
+    items, tiles = _plan_views(words, n_items.value)
+    _lib.check(lib.vdnh3_window_plan_build(
+        *geometry, bm, bn, ctypes.cast(items.data_ptr(), ctypes.POINTER(ctypes.c_int32)), n_items.value,
+        ctypes.cast(tiles.data_ptr(), ctypes.POINTER(ctypes.c_int32)), n_tiles.value), "window plan")
+    return items, tiles, int(pairs.value)
+
+
+def _plan_geometry(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames):
+    """The planner's geometry arguments."""
     if anchor_frames not in ANCHOR_FRAME_MODES:
         raise ValueError(f"anchor_frames={anchor_frames!r}; expected one of {ANCHOR_FRAME_MODES}")
     if len(bounds) != num_frames:
@@ -97,21 +117,13 @@ def build_plan_host(seq, video_start, video_end, num_frames, tokens_per_frame, b
     for frame, pair in enumerate(bounds):
         if len(pair) != 2:
             raise ValueError(f"bounds[{frame}] must be a (lo, hi) pair")
-    lib = _lib.lib()
     flat = (ctypes.c_int32 * max(1, 2 * num_frames))(*[int(x) for pair in bounds for x in pair])
-    bm, bn = lib.vdnh3_window_block_m(), lib.vdnh3_window_block_n()
-    mode = _lib.ANCHOR_MODE_CODES[anchor_frames]
-    n_items, n_tiles, pairs = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
-    _lib.check(lib.vdnh3_window_plan_size(int(seq), int(video_start), int(video_end), int(num_frames),
-                                          int(tokens_per_frame), flat, mode, bm, bn, ctypes.byref(n_items),
-                                          ctypes.byref(n_tiles), ctypes.byref(pairs)), "window plan")
-    items = torch.empty((n_items.value, 4), dtype=torch.int32)
-    tiles = torch.empty((n_tiles.value, 2), dtype=torch.int32)
-    _lib.check(lib.vdnh3_window_plan_build(
-        int(seq), int(video_start), int(video_end), int(num_frames), int(tokens_per_frame), flat, mode, bm, bn,
-        ctypes.cast(items.data_ptr(), ctypes.POINTER(ctypes.c_int32)), n_items.value,
-        ctypes.cast(tiles.data_ptr(), ctypes.POINTER(ctypes.c_int32)), n_tiles.value), "window plan")
-    return items, tiles, int(pairs.value)
+    return (int(seq), int(video_start), int(video_end), int(num_frames), int(tokens_per_frame), flat,
+            _lib.ANCHOR_MODE_CODES[anchor_frames])
+
+
+def _plan_views(words, n_items):
+    return words[:4 * n_items].view(n_items, 4), words[4 * n_items:].view(-1, 2)
 
 
 class WindowAttentionCache:
@@ -124,14 +136,16 @@ class WindowAttentionCache:
         self._plans: OrderedDict[tuple[Any, ...], WindowPlan] = OrderedDict()
         self.last_dispatch_reason: str | None = None
 
-    def plan(self, seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device):
+    def plan(self, seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device,
+             heads=None, dim=None):
         key = (int(seq), int(video_start), int(video_end), int(num_frames), int(tokens_per_frame),
-               tuple((int(a), int(b)) for a, b in bounds), str(anchor_frames), device.type, device.index)
+               tuple((int(a), int(b)) for a, b in bounds), str(anchor_frames), device.type, device.index, heads, dim)
         cached = self._plans.get(key)
         if cached is not None:
             self._plans.move_to_end(key)
             return cached
-        plan = make_plan(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device)
+        plan = make_plan(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device,
+                         heads, dim)
         self._plans[key] = plan
         while len(self._plans) > self.limit:
             self._plans.popitem(last=False)
@@ -147,10 +161,20 @@ class WindowAttentionCache:
         return len(self._plans)
 
 
-def make_plan(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device):
-    items, tiles, pairs = build_plan_host(seq, video_start, video_end, num_frames, tokens_per_frame, bounds,
-                                          anchor_frames)
-    return WindowPlan(items.to(device), tiles.to(device), items.shape[0], tiles.shape[0], pairs)
+def make_plan(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device, heads=None,
+              dim=None):
+    """The tile plan of a geometry; with ``heads`` and ``dim`` its items' height and key splits suit a call with that
+    many heads (``vdnh3_window_plan_shape``), without them items are whole and of the kernel's block height."""
+    geometry = (seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames)
+    block_m, splits = ctypes.c_int32(256), ctypes.c_int32(1)
+    if heads is not None:
+        lib = _lib.lib()
+        _lib.check(lib.vdnh3_window_plan_shape(*_plan_geometry(*geometry), lib.vdnh3_window_block_n(), int(heads),
+                                               int(dim), ctypes.byref(block_m), ctypes.byref(splits)), "window plan")
+    items, tiles, pairs = build_plan_host(*geometry, block_m.value)
+    n = items.shape[0]
+    words = torch.as_strided(items, (4 * n + tiles.numel(),), (1,)).to(device)
+    return WindowPlan(*_plan_views(words, n), n, tiles.shape[0], pairs, block_m.value, splits.value)
 
 
 def dense_plan(seq, device):
@@ -189,7 +213,8 @@ def _attention_operands(shape, device, plan, cache, geometry, gate, out):
     bf16 ``[S, H]`` view with unit head stride, and the output buffer (new or checked)."""
     seq, heads, dim = shape
     if plan is None:
-        plan = (cache.plan(*geometry, device) if cache is not None else make_plan(*geometry, device))
+        plan = (cache.plan(*geometry, device, heads, dim) if cache is not None
+                else make_plan(*geometry, device, heads, dim))
     if out is None:
         out = torch.empty((seq, heads, dim), dtype=torch.bfloat16, device=device)
     elif out.shape != (seq, heads, dim) or out.dtype != torch.bfloat16 or out.stride(2) != 1:
@@ -203,6 +228,15 @@ def _attention_operands(shape, device, plan, cache, geometry, gate, out):
             gate = gate.contiguous()
         g_row = gate.stride(0)
     return plan, gate, g_row, out
+
+
+def _partials(plan, heads, seq, dim, device):
+    """``(splits, buffer or None, its bytes)`` of a call with the plan's key splits."""
+    splits = plan.splits
+    if splits == 1:
+        return 1, None, 0
+    size = _lib.lib().vdnh3_window_partial_bytes(seq, heads, dim, splits)
+    return splits, torch.empty(size, dtype=torch.uint8, device=device), size
 
 
 def _check_qkv(query, key, value, name):
@@ -266,7 +300,8 @@ def window_softmax_hip(query, key, value, video_start, video_end, num_frames, to
     ws_bytes = lib.vdnh3_window_workspace_bytes(seq, heads, dim)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
     sh = _lib.stream_handle(device)
-    if diagnostics is None:
+    splits, partial, partial_bytes = _partials(plan, heads, seq, dim, device)
+    if diagnostics is None and splits == 1:
         rc = lib.vdnh3_window_attn_fwd(
             _lib.ptr(q), q.stride(0), q.stride(1), _lib.ptr(k), k.stride(0), k.stride(1),
             _lib.ptr(v), v.stride(0), v.stride(1), _lib.ptr(out), out.stride(0), out.stride(1),
@@ -274,15 +309,16 @@ def window_softmax_hip(query, key, value, video_start, video_end, num_frames, to
             _lib.ptr(plan.items), plan.n_items, _lib.ptr(plan.tiles), _lib.ptr(workspace), ws_bytes, sh)
         _lib.check(rc, "window_softmax_hip")
         return out
-    with diagnostics.scope("attention.softmax.vt_prepass", device):
+    with _maybe_scope(diagnostics, "attention.softmax.vt_prepass", device):
         rc = lib.vdnh3_window_vt_prepass(_lib.ptr(v), v.stride(0), v.stride(1), seq, heads, dim,
                                          _lib.ptr(workspace), ws_bytes, sh)
     _lib.check(rc, "window_softmax_hip")
-    with diagnostics.scope("attention.softmax.kernel", device):
-        rc = lib.vdnh3_window_attn_prepared(
+    with _maybe_scope(diagnostics, "attention.softmax.kernel", device):
+        rc = lib.vdnh3_window_attn_prepared_split(
             _lib.ptr(q), q.stride(0), q.stride(1), _lib.ptr(k), k.stride(0), k.stride(1),
             _lib.ptr(out), out.stride(0), out.stride(1), _lib.ptr(gate), g_row, seq, heads, dim, float(scale),
-            _lib.ptr(plan.items), plan.n_items, _lib.ptr(plan.tiles), _lib.ptr(workspace), ws_bytes, sh)
+            _lib.ptr(plan.items), plan.n_items, _lib.ptr(plan.tiles), _lib.ptr(workspace), ws_bytes, splits,
+            _lib.ptr(partial), partial_bytes, sh)
     _lib.check(rc, "window_softmax_hip")
     return out
 
@@ -319,6 +355,7 @@ def window_softmax_normed(q_raw, k_raw, value, q_weight, k_weight, q_eps, k_eps,
     ws_bytes = lib.vdnh3_window_norm_workspace_bytes(seq, heads, dim, int(rotate))
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
     sh = _lib.stream_handle(device)
+    splits, partial, partial_bytes = _partials(plan, heads, seq, dim, device)
     with _maybe_scope(diagnostics, "attention.softmax.qkv_prepass", device):
         rc = lib.vdnh3_window_qkv_prepass(
             _lib.ptr(q) if rotate else None, q.stride(0), q.stride(1), _lib.ptr(wq), float(q_eps),
@@ -331,16 +368,17 @@ def window_softmax_normed(q_raw, k_raw, value, q_weight, k_weight, q_eps, k_eps,
             region = lib.vdnh3_window_workspace_bytes(seq, heads, dim)
             head_stride = region // (2 * heads)
             base = workspace.data_ptr()
-            rc = lib.vdnh3_window_attn_prepared(
+            rc = lib.vdnh3_window_attn_prepared_split(
                 ctypes.c_void_p(base + 2 * region), dim, head_stride, ctypes.c_void_p(base + region), dim,
                 head_stride, _lib.ptr(out), out.stride(0), out.stride(1), _lib.ptr(gate), g_row, seq, heads, dim,
                 float(scale), _lib.ptr(plan.items), plan.n_items, _lib.ptr(plan.tiles), _lib.ptr(workspace),
-                ws_bytes, sh)
+                ws_bytes, splits, _lib.ptr(partial), partial_bytes, sh)
         else:
-            rc = lib.vdnh3_window_attn_qnorm(
+            rc = lib.vdnh3_window_attn_qnorm_split(
                 _lib.ptr(q), q.stride(0), q.stride(1), _lib.ptr(wq), float(q_eps),
                 _lib.ptr(out), out.stride(0), out.stride(1), _lib.ptr(gate), g_row, seq, heads, dim, float(scale),
-                _lib.ptr(plan.items), plan.n_items, _lib.ptr(plan.tiles), _lib.ptr(workspace), ws_bytes, sh)
+                _lib.ptr(plan.items), plan.n_items, _lib.ptr(plan.tiles), _lib.ptr(workspace), ws_bytes, splits,
+                _lib.ptr(partial), partial_bytes, sh)
     _lib.check(rc, "window_softmax_normed")
     return out
 

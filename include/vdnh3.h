@@ -69,6 +69,11 @@ int vdnh3_window_plan_build(int seq, int video_start, int video_end, int num_fra
                             int block_m, int block_n, int32_t *items, int32_t n_items,
                             int32_t *tiles, int32_t n_tiles);
 
+/* The item height (block_m: 256, 128 or 64 rows) and the number of key splits that suit a call with `heads` heads. */
+int vdnh3_window_plan_shape(int seq, int video_start, int video_end, int num_frames, int tokens_per_frame,
+                            const int32_t *bounds, int anchor_mode, int block_n, int heads, int head_dim,
+                            int32_t *block_m, int32_t *splits);
+
 /* Query/key tile sizes the attention kernel was built for. */
 int vdnh3_window_block_m(void);
 int vdnh3_window_block_n(void);
@@ -116,6 +121,21 @@ int vdnh3_window_attn_prepared(const uint16_t *q, int64_t q_row, int64_t q_head,
                                const void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * The same with each work item's key tiles divided over `splits` workgroups (1 to 64, and at most the smallest
+ * tile count of an item), whose partial results are combined by a second kernel: for calls with too few work
+ * items to fill the GPU. `partial` holds vdnh3_window_partial_bytes (unused with splits = 1).
+ */
+size_t vdnh3_window_partial_bytes(int seq, int heads, int head_dim, int splits);
+int vdnh3_window_attn_prepared_split(const uint16_t *q, int64_t q_row, int64_t q_head,
+                               const uint16_t *k, int64_t k_row, int64_t k_head,
+                               uint16_t *out, int64_t o_row, int64_t o_head,
+                               const uint16_t *gate, int64_t gate_row,
+                               int seq, int heads, int head_dim, float scale,
+                               const int32_t *items, int32_t n_items, const int32_t *tiles,
+                               const void *workspace, size_t workspace_bytes, int splits,
+    float *partial, size_t partial_bytes, void *stream);
+
+/*
  * The attention with the block's q_norm / k_norm fused in (vdn_h3/hybrid.py:271-292 followed by
  * the window softmax of vdn_h3/hybrid.py:295-302): q and k are passed raw, as the qkv projection
  * wrote them, and normalised with the arithmetic of vdnh3_qk_rmsnorm / vdnh3_qk_rmsnorm_rope, so
@@ -144,6 +164,13 @@ int vdnh3_window_attn_qnorm(const uint16_t *q, int64_t q_row, int64_t q_head, co
                             uint16_t *out, int64_t o_row, int64_t o_head, const uint16_t *gate, int64_t gate_row,
                             int seq, int heads, int head_dim, float scale, const int32_t *items, int32_t n_items,
                             const int32_t *tiles, const void *workspace, size_t workspace_bytes, void *stream);
+
+/* vdnh3_window_attn_qnorm with split key tiles (see vdnh3_window_attn_prepared_split). */
+int vdnh3_window_attn_qnorm_split(const uint16_t *q, int64_t q_row, int64_t q_head, const uint16_t *q_weight, float q_eps,
+                            uint16_t *out, int64_t o_row, int64_t o_head, const uint16_t *gate, int64_t gate_row,
+                            int seq, int heads, int head_dim, float scale, const int32_t *items, int32_t n_items,
+                            const int32_t *tiles, const void *workspace, size_t workspace_bytes, int splits,
+    float *partial, size_t partial_bytes, void *stream);
 
 /* ------------------------------------------------------------------------------
  * Projections (reference vdn_h3/projection.py, vdn_h3/fp8.py, the block's qkv/out GEMMs)

@@ -68,3 +68,22 @@ def test_plan_validation_errors(built_lib):
         window.build_plan_host(40, 4, 33, 3, 10, window.window_bounds(3, 1), "none")
     with pytest.raises(ValueError, match="anchor_frames"):
         window.build_plan_host(40, 4, 34, 3, 10, window.window_bounds(3, 1), "sideways")
+
+
+@pytest.mark.parametrize("heads", [1, 2, 7, 40])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("text,frames,per_frame", [(16, 13, 64), (1, 1, 1), (300, 20, 320), (512, 1, 1296), (512, 31, 1296)])
+def test_item_height_and_key_splits_rule(built_lib, heads, dim, text, frames, per_frame):
+    """The rule keeps to the kernel's limits, and a call that fills the 256 CUs several times over is left whole."""
+    from vdn_h3_amd import window
+
+    seq = text + frames * per_frame
+    geometry = (seq, text, seq, frames, per_frame, wo.window_bounds(frames, 1, 5), "both")
+    plan = window.make_plan(*geometry, torch.device("cpu"), heads, dim)
+    counts, rows = plan.items[:, 3], plan.items[:, 1] - plan.items[:, 0]
+    assert plan.block_m in (64, 128, 256) and int(rows.max()) <= plan.block_m and int(rows.sum()) == seq
+    assert 1 <= plan.splits <= int(counts.min())
+    if -(-seq // 256) * heads >= 1024:
+        assert (plan.block_m, plan.splits) == (256, 1)
+    whole = window.make_plan(*geometry, torch.device("cpu"))
+    assert (whole.block_m, whole.splits, whole.pairs_per_head) == (256, 1, plan.pairs_per_head)

@@ -180,3 +180,31 @@ def test_calls_hold_no_memory_beyond_their_output(device):
     grown = torch.cuda.memory_allocated(device) - base
     assert grown == kept.untyped_storage().nbytes() or grown == -(-kept.untyped_storage().nbytes() // 512) * 512
     assert torch.equal(kept, first)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("block_m,splits", [(256, 2), (256, 3), (128, 1), (128, 5), (64, 1), (64, 4), (256, "all")])
+def test_key_splits_and_short_items(device, dim, block_m, splits):
+    """Every item height and any number of key splits, up to one tile each, against the oracle, with and without a gate."""
+    from vdn_h3_amd import window
+
+    frames, per_frame, text, heads = 9, 61, 37, 3  # ragged: items of 37, 61 and 305 rows, masked tile edges
+    seq = text + frames * per_frame
+    bounds = wo.window_bounds(frames, 1, 4)
+    print(f"case splits D={dim} block_m={block_m} splits={splits}", flush=True)
+    geometry = (seq, text, seq, frames, per_frame, bounds, "both")
+    items, tiles, pairs = window.build_plan_host(*geometry, block_m)
+    fewest = int(items[:, 3].min())
+    assert int((items[:, 1] - items[:, 0]).max()) <= block_m and fewest >= 5
+    plan = window.WindowPlan(items.to(device), tiles.to(device), items.shape[0], tiles.shape[0], pairs, block_m,
+                             fewest if splits == "all" else splits)
+    gen = torch.Generator().manual_seed(17)
+    q, k, v = (torch.randn(seq, heads, dim, generator=gen).to(torch.bfloat16) for _ in range(3))
+    gate = torch.sigmoid(torch.randn(seq, heads, generator=gen)).to(torch.bfloat16)
+    want = wo.window_attention_grouped(q, k, v, *geometry[1:6], dim ** -0.5, "both")
+    args = (q.to(device), k.to(device), v.to(device), *geometry[1:6], dim ** -0.5, "both")
+    out = window.window_softmax_hip(*args, plan=plan)
+    gated = window.window_softmax_hip(*args, plan=plan, gate=gate.to(device))
+    torch.cuda.synchronize()
+    assert_parity(out, want)
+    assert torch.equal(gated, out * gate.to(device)[..., None])
