@@ -159,16 +159,15 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(message)
 
 
-def ptr(tensor) -> ctypes.c_void_p | None:
+def ptr(tensor) -> int | None:
     """Device (or host) address of a tensor, ``None`` for ``None``."""
-    if tensor is None:
-        return None
-    return ctypes.c_void_p(tensor.data_ptr())
+    return None if tensor is None else tensor.data_ptr()
 
 
-def stream_handle(device: torch.device) -> ctypes.c_void_p:
-    """Raw hipStream_t of torch's current stream on ``device``."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def stream_handle(device: torch.device) -> int:
+    """Raw hipStream_t of torch's current stream on ``device`` (0.3 us; through a ``Stream`` object 2 us)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def forward_only(what: str, *tensors) -> None:

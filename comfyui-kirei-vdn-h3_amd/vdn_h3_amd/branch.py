@@ -45,9 +45,9 @@ class _CholeskyChecks:
         if not self.statuses:
             return
         info = torch.cat([s.reshape(-1) for s in self.statuses])
-        bad = torch.nonzero(info != 0)
-        if bad.numel():
-            failed = int(bad[0, 0])
+        # one reduction and one host read on the way that always runs; the search only after a failure
+        if bool(info.any()):
+            failed = int(torch.nonzero(info)[0, 0])
             for index, status in enumerate(self.statuses):
                 if failed < status.numel():
                     minor = int(status.reshape(-1)[failed])

@@ -139,7 +139,7 @@ class WindowAttentionCache:
     def plan(self, seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device,
              heads=None, dim=None):
         key = (int(seq), int(video_start), int(video_end), int(num_frames), int(tokens_per_frame),
-               tuple((int(a), int(b)) for a, b in bounds), str(anchor_frames), device.type, device.index, heads, dim)
+               tuple(map(tuple, bounds)), str(anchor_frames), device.type, device.index, heads, dim)
         cached = self._plans.get(key)
         if cached is not None:
             self._plans.move_to_end(key)
@@ -184,8 +184,8 @@ def dense_plan(seq, device):
 
 def _kernel_operand(t: torch.Tensor) -> torch.Tensor:
     """A view the kernel can read in place (16-byte aligned rows/heads), else a contiguous copy."""
-    ok = (t.stride(2) == 1 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0)
-    return t if ok else t.contiguous()
+    row, head, chan = t.stride()
+    return t if chan == 1 and row % 8 == 0 and head % 8 == 0 and t.data_ptr() % 16 == 0 else t.contiguous()
 
 
 def rope_table(rope_freqs: torch.Tensor, seq: int, head_dim: int, device) -> tuple[torch.Tensor, int, int]:
@@ -204,7 +204,9 @@ def rope_table(rope_freqs: torch.Tensor, seq: int, head_dim: int, device) -> tup
     rows = rope_freqs.numel() // (4 * half)
     if rows not in (1, seq):
         raise ValueError(f"rope_freqs holds {rows} row entries; expected 1 or {seq}")
-    table = rope_freqs.reshape(rows, half, 2, 2).to(device=device, dtype=torch.float32).contiguous()
+    table = rope_freqs.reshape(rows, half, 2, 2)
+    if table.dtype != torch.float32 or table.device != device or not table.is_contiguous():
+        table = table.to(device=device, dtype=torch.float32).contiguous()
     return table, (0 if rows == 1 else 4 * half), rot
 
 
@@ -342,8 +344,8 @@ def window_softmax_normed(q_raw, k_raw, value, q_weight, k_weight, q_eps, k_eps,
     _lib.forward_only("window_softmax_normed", q_raw, k_raw, value, q_weight, k_weight, rope_freqs, gate)
     device = _lib.require_device(q_raw, k_raw, value, q_weight, k_weight, gate, out)
     seq, heads, dim = q_raw.shape
-    wq = q_weight.to(torch.bfloat16).contiguous()
-    wk = k_weight.to(torch.bfloat16).contiguous()
+    wq, wk = (w if w.dtype == torch.bfloat16 and w.is_contiguous() else w.to(torch.bfloat16).contiguous()
+              for w in (q_weight, k_weight))
     if wq.numel() != dim or wk.numel() != dim:
         raise ValueError(f"q/k norm weights must have {dim} entries")
     table, f_row, rot = (None, 0, 0) if rope_freqs is None else rope_table(rope_freqs, seq, dim, device)
