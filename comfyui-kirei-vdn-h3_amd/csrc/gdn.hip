@@ -328,21 +328,21 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(
     f.g = Gi[ch * GdnWs<D>::G + lane];
   };
 
-  // state block of this wave: S[v = 32 sl + row][k = 32 wave + l32]
+  // state block of this wave, transposed: st[i] is S[v = 32 sl + l32][k = 32 wave + 8 (i / 4) + 4 gl + i % 4], so a
+  // lane's elements are runs of four k and the bf16 copy is four 8-byte LDS writes (sixteen 2-byte ones from
+  // the untransposed product)
   f32x16_t st = {};
   if (s_init) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int vr = 8 * (i >> 2) + 4 * gl + (i & 3);
-      st[i] = s_init[((int64_t)h * D + 32 * sl + vr) * D + 32 * wave + l32];
+      st[i] = s_init[((int64_t)h * D + 32 * sl + l32) * D + 32 * wave + 8 * (i >> 2) + 4 * gl + (i & 3)];
     }
   }
   auto write_sb = [&]() __device__ {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int vr = 8 * (i >> 2) + 4 * gl + (i & 3);
-      Sb[vr * KP + 32 * wave + l32] = f2bf(st[i]);
-    }
+    for (int i = 0; i < 16; i += 4)
+      *reinterpret_cast<u32x2_t *>(Sb + l32 * KP + 32 * wave + 2 * i + 4 * gl) =
+          u32x2_t{pack_bf2(st[i], st[i + 1]), pack_bf2(st[i + 2], st[i + 3])};
   };
   // this wave's LDS writes are done, then the barrier
   auto lds_barrier = [&]() __device__ {
@@ -356,7 +356,8 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(
     if (tok < T) st16(out + (int64_t)tok * o_row + (int64_t)h * o_head + 32 * sl + 8 * pc, val);
   };
 
-  // O of chunk c - 1 between its two halves: Q^ S^T (step c - 1), P U (step c)
+  // O of chunk c - 1 between its two halves: Q^ S^T (step c - 1), P U (step c); transposed, a lane's values
+  // are four dv columns of one token
   f32x4_t oprev[2] = {};
   // P U of the chunk whose P fragments are p and whose U is in Ut[b], onto oprev
   auto pu = [&](const u32x4_t (&p)[C / 32], int b) __device__ {
@@ -364,14 +365,14 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(
     for (int s = 0; s < C / 32; ++s)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
-        oprev[nb] = mfma_bf16_16x16x32(as_bf16x8(p[s]),
-                                       as_bf16x8(ld16(Ut[b] + (16 * nb + l16) * CP + 32 * s + 8 * g4)), oprev[nb]);
+        oprev[nb] = mfma_bf16_16x16x32(as_bf16x8(ld16(Ut[b] + (16 * nb + l16) * CP + 32 * s + 8 * g4)),
+                                       as_bf16x8(p[s]), oprev[nb]);
   };
   auto write_o = [&](int b) __device__ {
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Os[b][(16 * wave + 4 * g4 + i) * OP + 16 * nb + l16] = f2bf(oprev[nb][i]);
+      *reinterpret_cast<u32x2_t *>(Os[b] + (16 * wave + l16) * OP + 16 * nb + 4 * g4) =
+          u32x2_t{pack_bf2(oprev[nb][0], oprev[nb][1]), pack_bf2(oprev[nb][2], oprev[nb][3])};
   };
 
   // Step c computes chunk c from register set f; `ahead` holds chunk c - 1 until it is reloaded
@@ -395,8 +396,8 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(
     for (int s = 0; s < D / 32; ++s)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
-        ocur[nb] = mfma_bf16_16x16x32(as_bf16x8(f.q[s]),
-                                      as_bf16x8(ld16(Sb + (16 * nb + l16) * KP + 32 * s + 8 * g4)), ocur[nb]);
+        ocur[nb] = mfma_bf16_16x16x32(as_bf16x8(ld16(Sb + (16 * nb + l16) * KP + 32 * s + 8 * g4)),
+                                      as_bf16x8(f.q[s]), ocur[nb]);
     // U[tok][dv] = U~ - W S^T, stored transposed (Ut[dv][tok]): four consecutive tokens per write
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(
     for (int i = 0; i < 16; ++i) st[i] *= decay;
 #pragma unroll
     for (int s = 0; s < C / 16; ++s)
-      st = mfma_bf16_32x32x16(as_bf16x8(ld16(Ut[b] + l32 * CP + 16 * s + 8 * gl)), as_bf16x8(f.k[s]), st);
+      st = mfma_bf16_32x32x16(as_bf16x8(f.k[s]), as_bf16x8(ld16(Ut[b] + l32 * CP + 16 * s + 8 * gl)), st);
     write_sb();
     lds_barrier();
 #pragma unroll
@@ -446,8 +447,7 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(
   if (s_final) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int vr = 8 * (i >> 2) + 4 * gl + (i & 3);
-      s_final[((int64_t)h * D + 32 * sl + vr) * D + 32 * wave + l32] = st[i];
+      s_final[((int64_t)h * D + 32 * sl + l32) * D + 32 * wave + 8 * (i >> 2) + 4 * gl + (i & 3)] = st[i];
     }
   }
   wait_vm_lds<0>();  // the loads of the two chunks past the end land before the wave ends
