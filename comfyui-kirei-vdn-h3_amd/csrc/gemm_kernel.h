@@ -27,7 +27,8 @@
 // What bounds it: power, then the tile loads. At 8192^3 in bf16 the kernel takes 788 us (877 with the 32x32
 // shapes and 64-byte stages), 645 without its tile loads (timing only), 766 without its epilogue; the MFMA
 // pipes are busy 0.77 of the cycles at 1.67 GHz. At 40,688 x 15,360 x 5,120, alternated with that kernel
-// on one machine: int8 2422 us against 2812, fp8 2291 against 2664 (2642 and 2793 T(FL)OP/s).
+// on one machine: int8 2422 us against 2812, fp8 2291 against 2664 (2642 and 2793 T(FL)OP/s). Bands that start their
+// columns apart: 8192^3 bf16 775 -> 752 us, fp8 400 -> 380, int8 415 -> 393; 8,296 x 15,360 x 5,120 fp8 504 -> 487.
 #pragma once
 #include <type_traits>
 
@@ -306,7 +307,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_nt_kernel(const GemmArgs
   const int band = L / (kGroup * args.tiles_n);
   const int band_m = min(kGroup, args.tiles_m - band * kGroup);
   const int in_band = L - band * kGroup * args.tiles_n;
-  const int m0 = (band * kGroup + in_band % band_m) * BM, n0 = in_band / band_m * kGemmBN;
+  // A band starts its columns 5/8 of the way round from the last one's: the XCDs work on different bands, and
+  // starting on the same columns they would all fetch the same B panels from the same memory channels at once
+  const int column = (in_band / band_m + band * 5 * args.tiles_n / 8) % args.tiles_n;
+  const int m0 = (band * kGroup + in_band % band_m) * BM, n0 = column * kGemmBN;
 
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
