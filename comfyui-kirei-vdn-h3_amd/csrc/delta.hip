@@ -447,9 +447,19 @@ __global__ void alpha_logsum_kernel(const float *__restrict__ alpha, float *__re
   if (e >= hd) return;
   float lp = 0.f;
   out[e] = 0.f;
-  for (int i = 0; i < F; ++i) {
-    lp += logf(fmaxf(alpha[(int64_t)i * hd + e], 1e-12f));
-    out[(int64_t)(i + 1) * hd + e] = lp;
+  // eight frames' loads and logarithms at a time, then their sums in order (one load per sum was a chain of
+  // round trips: 35 frames of 5,120 18 us, so 7.4 us)
+  for (int i0 = 0; i0 < F; i0 += 8) {
+    float a[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = alpha[(int64_t)min(i0 + u, F - 1) * hd + e];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = logf(fmaxf(a[u], 1e-12f));
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      lp += a[u];
+      if (i0 + u < F) out[(int64_t)(i0 + u + 1) * hd + e] = lp;
+    }
   }
 }
 
