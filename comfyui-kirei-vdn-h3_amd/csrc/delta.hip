@@ -358,8 +358,8 @@ __global__ __launch_bounds__(256, 4) void factor_kernel(const FactorJob job0, co
 // The steps are a chain, their operands are not: a step loads the next one's Phi and J into a second register
 // set, eight loads after every eight products (all issued before the products they exceed the 63 operations
 // a wait can count, and the products waited for all of them; one load after each product was 30% slower).
-// Contraction index kappa = 8 (s / 4) + 4 g + s % 4 belongs to product s and lane group g, and the state lies
-// in LDS by (g, row, s), so a lane reads and writes it 16 bytes at a time. 40 heads of 128, 35 frames: 260 ->
+// Contraction index kappa = 2 s + g belongs to product s and lane group g, so that the products sum in ascending
+// order, and the state lies in LDS by (g, row, s), so a lane reads it 16 bytes at a time and writes it 8. 40 heads of 128, 35 frames: 260 ->
 // 219 us (176 without the loads: the 64 CUs that hold two of the 320 workgroups set the time); 8 heads, 11
 // frames: 53 -> 34 us; 13 heads of 64, 70 frames: 163 -> 94 us.
 template <int D>
@@ -378,13 +378,12 @@ __global__ __launch_bounds__(64 * (D / 32)) void scan_kernel(const float *__rest
   const int r0 = rb * 32;
   for (int e = tid; e < D * 32; e += 64 * NRB) {
     const int c = e >> 5, r = e & 31;
-    St[0][(c >> 2) & 1][r * PITCH + 4 * (c >> 3) + (c & 3)] =
-        init ? init[((int64_t)h * D + r0 + r) * D + c] : 0.f;
+    St[0][c & 1][r * PITCH + (c >> 1)] = init ? init[((int64_t)h * D + r0 + r) * D + c] : 0.f;
   }
   __syncthreads();
   float *out = dir == 0 ? prefix : suffix;
   const int64_t hd2 = (int64_t)h * D * D, frame = (int64_t)heads * D * D;
-  const uint32_t phi_lane = 4 * g * D + 32 * cb + l32;                      // + (s % 4) D
+  const uint32_t phi_lane = g * D + 32 * cb + l32;                           // + 2 (s % 4) D
   const int64_t row_lane = hd2 + (int64_t)(r0 + l32) * D + 32 * cb + 4 * g;  // + 8 i4: J and the output
   auto frame_of = [&](int step) __device__ { return (dir == 0 ? step : F - 1 - step) * frame; };
   struct Operands {
@@ -403,19 +402,20 @@ __global__ __launch_bounds__(64 * (D / 32)) void scan_kernel(const float *__rest
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       acc = mfma_f32_32x32x2(o.phi[s], x[s >> 2][s & 3], acc);
-      n.phi[s] = (Pn + 8 * (s >> 2) * D)[phi_lane + (s & 3) * D];
+      n.phi[s] = (Pn + 8 * (s >> 2) * D)[phi_lane + 2 * (s & 3) * D];
       if ((s & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) n.j[i4] = *reinterpret_cast<const f32x4_t *>(Jn + 8 * i4);
     float *Or = out + frame_of(step) + row_lane;
-    float *Y = St[(step & 1) ^ 1][g] + l32 * PITCH + 16 * cb;
+    float *Y = St[(step & 1) ^ 1][0] + l32 * PITCH + 16 * cb + 2 * g;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       f32x4_t r;
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[e] = acc[4 * i4 + e] + o.j[i4][e];
-      *reinterpret_cast<f32x4_t *>(Y + 4 * i4) = r;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) *reinterpret_cast<float2 *>(Y + e * 32 * PITCH + 4 * i4) = make_float2(r[e], r[e + 2]);
       *reinterpret_cast<f32x4_t *>(Or + 8 * i4) = r;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the state is in LDS; loads and stores stay in flight
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(64 * (D / 32)) void scan_kernel(const float *__rest
   {
     const float *P0 = Phi + frame_of(0) + hd2, *J0 = J + frame_of(0) + row_lane;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) o0.phi[s] = (P0 + 8 * (s >> 2) * D)[phi_lane + (s & 3) * D];
+    for (int s = 0; s < NS; ++s) o0.phi[s] = (P0 + 8 * (s >> 2) * D)[phi_lane + 2 * (s & 3) * D];
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) o0.j[i4] = *reinterpret_cast<const f32x4_t *>(J0 + 8 * i4);
   }

@@ -174,6 +174,22 @@ def test_scan_steps_and_item_counts(device, frames, heads, dim):
             assert bool((err <= frames * (dim + 1) * 2.0 ** -24 * bound).all()), (f, err.max().item())
 
 
+@pytest.mark.parametrize("frames,dim", [(1, 128), (4, 64)])
+def test_scan_sums_in_ascending_order(device, frames, dim):
+    """A step's products are added one after the other in ascending order of the contraction index, in fp32."""
+    from vdn_h3_amd import branch
+
+    heads = 2
+    spread = torch.exp(4 * _rand((frames, heads, dim, dim), 95))  # magnitudes far apart: another order rounds otherwise
+    phi, jay = _rand((frames, heads, dim, dim), 94) * spread, _rand((frames, heads, dim, dim), 96)
+    got = branch.run_scans_from_factors(phi.to(device), jay.to(device), torch.ones(heads, dim, dim, device=device))
+    for out, f in zip(got, (0, frames - 1)):  # the first step of each direction starts from ones: products are exact
+        acc = torch.zeros(heads, dim)
+        for k in range(dim):
+            acc = acc + phi[f, :, k]
+        assert torch.equal(out[f].cpu(), acc[:, None] + jay[f])
+
+
 @pytest.mark.parametrize("dim,k_features,v_features,a_fp32,text_rows", [
     (128, True, True, True, 33), (128, False, False, True, 1), (64, True, False, False, 64), (64, False, True, True, 200)])
 def test_text_state_shares_the_video_launches(device, dim, k_features, v_features, a_fp32, text_rows):
