@@ -43,9 +43,19 @@ constexpr int kRing = 3;  // LDS slots per K and V^T ring (144 KB at D = 128): l
 constexpr int kAhead = 4;
 constexpr float kLazy = 8.0f;  // log2 of the largest probability a stale running max allows
 
-// LDS position p (0..31) inside a 32-key group holds key offset kperm(p): the order in which lane
-// group g = p / 8 holds its 8 keys of a k-step in two 16x16 blocks of S^T.
-__host__ __device__ constexpr int kperm(int p) { return 16 * ((p & 7) >> 2) + 4 * (p >> 3) + (p & 3); }
+// LDS position p (0..31) of V^T inside a 32-key group holds key offset kperm(p): the order in which lane
+// group g = p / 8 holds its 8 keys of a k-step in two 16x16 blocks of S^T, whose rows are the K tile's LDS rows
+// r, holding keys krow(r). The keys of lane groups 0 and 1 are those of the group's first half, so the PV product
+// sums 16 keys before the next 16, bit for bit as 32x32x16 MFMAs do. Of the rounding only the row sums are
+// then left apart from that shape's: 2e-5 of the output in 2-norm at 16,007 x 56 x 128 (with a lane group's keys 16
+// apart 5e-5; a block's output 1.3e-5 to 2.5e-5 against 1.7e-4 to 2.4e-4). It costs nothing: the K tile loads
+// fetch their rows in this order.
+__host__ __device__ constexpr int kperm(int p) {
+  return 16 * (p >> 4) + 8 * ((p & 7) >> 2) + 4 * ((p >> 3) & 1) + (p & 3);
+}
+__host__ __device__ constexpr int krow(int r) {
+  return 32 * (r >> 5) + 16 * ((r >> 3) & 1) + 8 * ((r >> 4) & 1) + (r & 7);
+}
 
 // ---------------------------------------------------------------------------------
 // LDS slots of the staged tiles. Each tile row is split into 16-byte chunks; chunk c of row r
@@ -460,7 +470,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   const uint16_t *vbase = vt + (int64_t)head * D * s_pad;
   // Tile loads, by one group of 256 threads: thread chunk i fills LDS position P = 256 i + gtid
   // (16-byte units) of the tile. In a K tile, P is (row P / KC, slot P % KC) and holds chunk
-  // slot ^ swizzle(row) of that key row; row kr0 + i * 256 / KC has the same swizzle for every i.
+  // slot ^ swizzle(row) of key row krow(row); row kr0 + i * 256 / KC has the same swizzle for every i.
   // A V^T tile image is already in LDS order: P comes from position P of the image.
   // Rows past seq read row seq - 1 (their scores are masked).
   constexpr int KCG = kBN * KC / 256, VCG = D * (kBN / 8) / 256;  // 16-byte chunks per thread and tile
@@ -475,7 +485,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
 #pragma unroll
   for (int i = 0; i < KCG; ++i) {
     const int P = 256 * i + gtid;
-    doff[i] = 2u * (group == 0 ? (uint32_t)((kr0 + i * (256 / KC)) * (int)k_row + kslot) : (uint32_t)(P * 8));
+    doff[i] = 2u * (group == 0 ? (uint32_t)(krow(kr0 + i * (256 / KC)) * (int)k_row + kslot) : (uint32_t)(P * 8));
   }
   const uint32_t lds_dma = __builtin_amdgcn_readfirstlane(
       (group == 0 ? lds_address(&Ks[0][0]) : lds_address(&Vs[0][0])) + gw * 64 * 16);
@@ -491,7 +501,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
     if (group == 0 && ks + kBN > seq) {  // uniform: taken for the last tile of the sequence only
 #pragma unroll
       for (int i = 0; i < KCG; ++i)
-        off[i] = 2u * (uint32_t)((min(ks + kr0 + i * (256 / KC), seq - 1) - ks) * (int)k_row + kslot);
+        off[i] = 2u * (uint32_t)((min(ks + krow(kr0 + i * (256 / KC)), seq - 1) - ks) * (int)k_row + kslot);
     }
 #pragma unroll
     for (int i = 0; i < KCG; ++i)
@@ -621,7 +631,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
           for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const int ko = 16 * kb + 4 * g + i;
+              const int ko = krow(16 * kb) + krow(4 * g) + i;
               if (ko < lo || ko >= hi) {
 #pragma unroll
                 for (int n = 0; n < kNQ; ++n) sacc[kb][n][i] = -INFINITY;

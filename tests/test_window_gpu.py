@@ -208,3 +208,21 @@ def test_key_splits_and_short_items(device, dim, block_m, splits):
     torch.cuda.synchronize()
     assert_parity(out, want)
     assert torch.equal(gated, out * gate.to(device)[..., None])
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_values_sum_sixteen_keys_at_a_time(device, dim):
+    """The PV product adds the keys of one aligned group of 16 before those of the next: large values that cancel within
+    a group leave no rounding behind for a small one in the next group."""
+    from vdn_h3_amd import window
+
+    seq, heads = 192, 2
+    q = torch.zeros(seq, heads, dim, dtype=torch.bfloat16, device=device)  # equal scores: every probability is 1
+    v = torch.zeros_like(q)
+    for group in range(seq // 32):  # a channel per pair of groups
+        v[32 * group + 4, :, group], v[32 * group + 8, :, group], v[32 * group + 16, :, group] = 2.0 ** 30, -2.0 ** 30, 1
+    out = window.window_softmax_hip(q, q, v, 0, seq, 1, seq, [(0, 0)], dim ** -0.5, "none",
+                                    plan=window.dense_plan(seq, device))
+    want = torch.zeros_like(out)
+    want[..., :seq // 32] = 1 / seq
+    assert torch.equal(out, want)
