@@ -42,6 +42,11 @@ constexpr int kRing = 3;  // LDS slots per K and V^T ring (144 KB at D = 128): l
 // at the full shape, and with the row sums as MFMAs 6 / 5 / 4 15.04 / 15.09 / 15.02
 constexpr int kAhead = 4;
 constexpr float kLazy = 8.0f;  // log2 of the largest probability a stale running max allows
+// The running max before the first score above it. Finite, so that a tile whose scores are all -inf (keys masked
+// through a channel of q and k) adds zeros and not exp2(-inf + inf); and above every masked score of a type's
+// lowest value, whose rounded product with the scale is no maximum to subtract (its last place exceeds 2^128). A row
+// with no score above it has no sum: 0 / 0, NaN, as of a row of -inf.
+constexpr float kNoMax = -2147483648.0f;
 
 // LDS position p (0..31) of V^T inside a 32-key group holds key offset kperm(p): the order in which lane
 // group g = p / 8 holds its 8 keys of a k-step in two 16x16 blocks of S^T, whose rows are the K tile's LDS rows
@@ -528,7 +533,7 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
     for (int m = 0; m < NO; ++m) oacc[m][n] = f32x4_t{};
 #pragma unroll
     for (int j = 0; j < NT; ++j) pb[j][n] = u32x4_t{};
-    m_run[n] = -INFINITY;
+    m_run[n] = kNoMax;
     l_run[n] = f32x4_t{};
   }
 

@@ -226,3 +226,36 @@ def test_values_sum_sixteen_keys_at_a_time(device, dim):
     want = torch.zeros_like(out)
     want[..., :seq // 32] = 1 / seq
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("value", [float("-inf"), torch.finfo(torch.bfloat16).min, -1e9])
+@pytest.mark.parametrize("block_m,splits", [(256, 1), (256, 3), (64, 4), (256, "all")])
+def test_masked_tiles_add_nothing(device, dim, value, block_m, splits):
+    """Keys masked through a channel of q and k, whole key tiles of them: at the front of an item's or of a split's tiles
+    too, they take no part, and a row with no other key is NaN."""
+    from vdn_h3_amd import window
+
+    frames, per_frame, text, heads = 9, 192, 192, 2  # 96-key tiles: two to a frame
+    seq = text + frames * per_frame
+    geometry = (seq, text, seq, frames, per_frame, wo.window_bounds(frames, 1), "both")
+    items, tiles, pairs = window.build_plan_host(*geometry, block_m)
+    fewest = int(items[:, 3].min())
+    plan = window.WindowPlan(items.to(device), tiles.to(device), items.shape[0], tiles.shape[0], pairs, block_m,
+                             fewest if splits == "all" else splits)
+    gen = torch.Generator().manual_seed(19)
+    q, k, v = (torch.randn(seq, heads, dim, generator=gen).to(torch.bfloat16) for _ in range(3))
+    q[..., -1], k[..., -1] = 1, 0
+    k[:96, :, -1] = value   # the first tile of every item
+    for frame in (2, 4):    # the first tiles of a split, in three splits of the rows of frames 0 (20 tiles) and 5 (12)
+        k[text + frame * 192:text + (frame + 1) * 192, :, -1] = value
+    k[-96:, 1, -1] = value  # the last tile, of one head
+    want = wo.window_attention_grouped(q, k, v, *geometry[1:6], dim ** -0.5, "both")
+    assert bool(want.isfinite().all())
+    args = (*geometry[1:6], dim ** -0.5, "both")
+    out = window.window_softmax_hip(q.to(device), k.to(device), v.to(device), *args, plan=plan)
+    assert_parity(out, want)
+    if value == float("-inf"):
+        k[..., -1] = value
+        out = window.window_softmax_hip(q.to(device), k.to(device), v.to(device), *args, plan=plan)
+        assert bool(out.isnan().all())
