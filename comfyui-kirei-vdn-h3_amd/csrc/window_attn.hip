@@ -456,11 +456,20 @@ __global__ __launch_bounds__(kThreads, 1) void window_attn_kernel(
   if (L >= total) return;
   const int head = L / n_items;
   const int4 item = items[L - head * n_items];
-  // grid.y splits of the item's key tiles (the host keeps it at or below every item's tile count)
+  // grid.y splits of the item's key tiles
   const int t0 = item.w * (int)blockIdx.y / (int)gridDim.y, t1 = item.w * ((int)blockIdx.y + 1) / (int)gridDim.y;
   const int q0 = item.x, q1 = item.y, toff = item.z + t0, T = t1 - t0;
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (T == 0) {  // more splits than the item has tiles: this one adds nothing
+    if (part.o) {
+      const int64_t row = ((int64_t)blockIdx.y * (total / n_items) + head) * seq + q0;
+      for (int e = tid; e < (q1 - q0) * D; e += kThreads) part.o[row * D + e] = 0.f;
+      for (int r = tid; r < q1 - q0; r += kThreads)
+        *reinterpret_cast<float2 *>(part.ml + (row + r) * 2) = make_float2(kNoMax, 0.f);
+    }
+    return;
+  }
   const int l16 = lane & 15, g = lane >> 4;
   const int group = wave >> 2;
   // a wavefront whose 32 rows all lie past the item's end (the short last item of a run) skips

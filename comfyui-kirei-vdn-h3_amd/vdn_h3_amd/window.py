@@ -87,7 +87,7 @@ class WindowPlan:
     n_tiles: int
     pairs_per_head: int     # allowed (query, key) pairs per head
     block_m: int = 256      # most query rows of an item
-    splits: int = 1         # workgroups that divide an item's key tiles (at most its fewest tiles)
+    splits: int = 1         # workgroups that divide an item's key tiles (past its tile count they add nothing)
 
 
 def build_plan_host(seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, block_m=None):

@@ -121,8 +121,8 @@ int vdnh3_window_attn_prepared(const uint16_t *q, int64_t q_row, int64_t q_head,
                                const void *workspace, size_t workspace_bytes, void *stream);
 
 /*
- * The same with each work item's key tiles divided over `splits` workgroups (1 to 64, and at most the smallest
- * tile count of an item), whose partial results are combined by a second kernel: for calls with too few work
+ * The same with each work item's key tiles divided over `splits` workgroups (1 to 64; those past an item's tile
+ * count add nothing), whose partial results are combined by a second kernel: for calls with too few work
  * items to fill the GPU. `partial` holds vdnh3_window_partial_bytes (unused with splits = 1).
  */
 size_t vdnh3_window_partial_bytes(int seq, int heads, int head_dim, int splits);

@@ -259,3 +259,25 @@ def test_masked_tiles_add_nothing(device, dim, value, block_m, splits):
         k[..., -1] = value
         out = window.window_softmax_hip(q.to(device), k.to(device), v.to(device), *args, plan=plan)
         assert bool(out.isnan().all())
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_more_splits_than_tiles(device, dim):
+    """The splits past an item's tile count read no tile and add nothing; items of the same plan differ in count."""
+    from vdn_h3_amd import window
+
+    frames, per_frame, text, heads = 9, 61, 37, 3
+    seq = text + frames * per_frame
+    geometry = (seq, text, seq, frames, per_frame, wo.window_bounds(frames, 1), "columns")
+    items, tiles, pairs = window.build_plan_host(*geometry, 64)
+    counts = items[:, 3]
+    assert int(counts.min()) < int(counts.max()) < 64
+    gen = torch.Generator().manual_seed(29)
+    q, k, v = (torch.randn(seq, heads, dim, generator=gen).to(torch.bfloat16) for _ in range(3))
+    want = wo.window_attention_grouped(q, k, v, *geometry[1:6], dim ** -0.5, "columns")
+    for splits in (int(counts.min()) + 1, 64):
+        print(f"case splits past the tiles D={dim} splits={splits}", flush=True)
+        plan = window.WindowPlan(items.to(device), tiles.to(device), items.shape[0], tiles.shape[0], pairs, 64, splits)
+        out = window.window_softmax_hip(q.to(device), k.to(device), v.to(device), *geometry[1:6], dim ** -0.5, "columns",
+                                        plan=plan)
+        assert_parity(out, want)
