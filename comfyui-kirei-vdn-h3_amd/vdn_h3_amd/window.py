@@ -122,6 +122,14 @@ def _plan_geometry(seq, video_start, video_end, num_frames, tokens_per_frame, bo
             _lib.ANCHOR_MODE_CODES[anchor_frames])
 
 
+def _bounds_key(bounds):
+    """The bounds as tuples of ints, whatever holds them: tensors hash by identity and would miss the cache every call."""
+    pairs = tuple(map(tuple, bounds))
+    if pairs and set(map(type, pairs[0])) == {int}:  # the geometry's own; asking of every pair takes as long again
+        return pairs
+    return tuple((int(lo), int(hi)) for lo, hi in pairs)
+
+
 def _plan_views(words, n_items):
     return words[:4 * n_items].view(n_items, 4), words[4 * n_items:].view(-1, 2)
 
@@ -139,7 +147,7 @@ class WindowAttentionCache:
     def plan(self, seq, video_start, video_end, num_frames, tokens_per_frame, bounds, anchor_frames, device,
              heads=None, dim=None):
         key = (int(seq), int(video_start), int(video_end), int(num_frames), int(tokens_per_frame),
-               tuple(map(tuple, bounds)), str(anchor_frames), device.type, device.index, heads, dim)
+               _bounds_key(bounds), str(anchor_frames), device.type, device.index, heads, dim)
         cached = self._plans.get(key)
         if cached is not None:
             self._plans.move_to_end(key)

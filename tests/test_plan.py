@@ -87,3 +87,19 @@ def test_item_height_and_key_splits_rule(built_lib, heads, dim, text, frames, pe
         assert (plan.block_m, plan.splits) == (256, 1)
     whole = window.make_plan(*geometry, torch.device("cpu"))
     assert (whole.block_m, whole.splits, whole.pairs_per_head) == (256, 1, plan.pairs_per_head)
+
+
+@pytest.mark.parametrize("hold", [list, tuple, torch.tensor, lambda b: torch.tensor(b).numpy(),
+                                  lambda b: [torch.tensor(p) for p in b]])
+def test_cached_plan_whatever_holds_the_bounds(built_lib, hold):
+    from vdn_h3_amd import window
+
+    bounds = wo.window_bounds(5, 1, 2)
+    cache, device = window.WindowAttentionCache(), torch.device("cpu")
+    geometry = lambda b: (516, 16, 516, 5, 100, b, "both", device, 2, 64)  # noqa: E731
+    first = cache.plan(*geometry(bounds))
+    assert cache.plan(*geometry(hold(bounds))) is first
+    assert cache.plan(*geometry(hold(bounds))) is first and len(cache) == 1
+    for wrong in ([(0, 1, 2), (3,)], [(0,)] * 5, []):
+        with pytest.raises(ValueError):
+            cache.plan(*geometry(wrong))
