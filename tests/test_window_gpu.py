@@ -281,3 +281,38 @@ def test_more_splits_than_tiles(device, dim):
         out = window.window_softmax_hip(q.to(device), k.to(device), v.to(device), *geometry[1:6], dim ** -0.5, "columns",
                                         plan=plan)
         assert_parity(out, want)
+
+
+@pytest.mark.parametrize("normed", [False, True])
+def test_items_stay_whole_without_memory_for_partials(device, monkeypatch, normed):
+    """A call whose partial results find no memory runs its items whole: the result of the same plan without splits."""
+    from dataclasses import replace
+
+    from vdn_h3_amd import _lib, window
+
+    seq, heads, dim = 700, 2, 128
+    plan = replace(window.dense_plan(seq, device), splits=3)
+    size = _lib.lib().vdnh3_window_partial_bytes(seq, heads, dim, 3)
+    gen = torch.Generator().manual_seed(31)
+    q, k, v = (torch.randn(seq, heads, dim, generator=gen).to(torch.bfloat16).to(device) for _ in range(3))
+    weight = torch.ones(dim, dtype=torch.bfloat16, device=device)
+
+    def call(plan):
+        geometry = (0, seq, 1, seq, [(0, 0)])
+        if normed:
+            return window.window_softmax_normed(q, k, v, weight, weight, 1e-6, 1e-6, *geometry, dim ** -0.5, "none",
+                                                plan=plan)
+        return window.window_softmax_hip(q, k, v, *geometry, dim ** -0.5, "none", plan=plan)
+
+    whole, split, empty = call(replace(plan, splits=1)), call(plan), torch.empty
+    refused = []
+
+    def full(*shape, **options):
+        if shape[0] == size:
+            refused.append(size)
+            raise torch.OutOfMemoryError("out of memory")
+        return empty(*shape, **options)
+
+    monkeypatch.setattr(torch, "empty", full)
+    out = call(plan)
+    assert refused and torch.equal(out, whole) and not torch.equal(split, whole)
