@@ -164,10 +164,16 @@ def ptr(tensor) -> int | None:
     return None if tensor is None else tensor.data_ptr()
 
 
+# not part of torch's public interface: a build without it takes the public way below
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device: torch.device) -> int:
     """Raw hipStream_t of torch's current stream on ``device`` (0.3 us; through a ``Stream`` object 2 us)."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def forward_only(what: str, *tensors) -> None:

@@ -199,3 +199,20 @@ def test_readout_frame_range_checks():
             branch.readout_epilogue(q, banks, banks, alpha, bounds, torch.ones(dim), None, frame_range=bad, **kw)
     with pytest.raises(ValueError, match="range's frames"):
         branch.readout_epilogue(q, banks, banks, alpha, bounds, torch.ones(dim), None, frame_range=(0, 3), **kw)
+
+
+def test_stream_handle_without_the_private_call(monkeypatch):
+    """A torch build without the raw-stream call gives the handle through its public interface."""
+    import importlib
+    from types import SimpleNamespace
+
+    from vdn_h3_amd import _lib
+
+    private = SimpleNamespace(**{n: getattr(torch._C, n) for n in dir(torch._C) if n != "_cuda_getCurrentRawStream"})
+    with monkeypatch.context() as m:
+        m.setattr(torch, "_C", private)
+        m.setattr(torch.cuda, "current_stream", lambda device: SimpleNamespace(cuda_stream=77))
+        spec = importlib.util.spec_from_file_location("vdn_h3_amd._lib_without", _lib.__file__)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        assert module.stream_handle(torch.device("cuda", 0)) == 77
