@@ -86,19 +86,26 @@ __device__ __forceinline__ constexpr int gemm_slot(int r, int c) { return c ^ ((
 // Output stores, and the loads of the old values when accumulating, are non-temporal (the `nt`
 // hint): the output streams through each XCD's L2 at 128 KB per tile, which would otherwise
 // evict the A and B panels that the XCD's other workgroups are still reading.
-template <typename V, typename P>
-__device__ __forceinline__ void stream_store(V v, P *p) {
-  __builtin_nontemporal_store(v, reinterpret_cast<V *>(p));
-}
-template <typename V, typename P>
-__device__ __forceinline__ V stream_load(const P *p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const V *>(p));
-}
-// 16 bytes of C at the alignment of its elements (any N and ldc; global accesses of any alignment are one
-// instruction here)
+// C is aligned to its elements only (any N and ldc; global accesses of any alignment are one instruction here), and
+// the pointers say so: the types are no template arguments, which would lose their alignment.
 typedef u32x4_t __attribute__((aligned(2))) u32x4_a2_t;
 typedef u32x4_t __attribute__((aligned(4))) u32x4_a4_t;
 typedef f32x4_t __attribute__((aligned(4))) f32x4_a4_t;
+__device__ __forceinline__ void stream_store(u32x4_t v, uint16_t *p) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a2_t *>(p));
+}
+__device__ __forceinline__ void stream_store(u32x4_t v, int32_t *p) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a4_t *>(p));
+}
+__device__ __forceinline__ void stream_store(f32x4_t v, float *p) {
+  __builtin_nontemporal_store(v, reinterpret_cast<f32x4_a4_t *>(p));
+}
+__device__ __forceinline__ u32x4_t stream_load(const uint16_t *p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2_t *>(p));
+}
+__device__ __forceinline__ f32x4_t stream_load(const float *p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4_t *>(p));
+}
 
 // Epilogue operands. Loaded at the start of the kernel, one column (its scale times alpha, its bias) and
 // MI / 4 rows per lane, so that their latency hides behind the main loop at 2 + MI / 4 registers; the
@@ -183,7 +190,7 @@ __device__ __forceinline__ void store_block(const Acc (&acc)[MI][4], float *stag
 #pragma unroll
           for (int r = 0; r < 2; ++r)
             if (i0 + b < MI && n + 8 <= N && m0 + 16 * (i0 + b) + r < M)
-              old[b][r] = stream_load<u32x4_a2_t>(cp + (int64_t)(16 * (i0 + b) + r) * ldc);
+              old[b][r] = stream_load(cp + (int64_t)(16 * (i0 + b) + r) * ldc);
       }
 #pragma unroll
       for (int b = 0; b < kBatch; ++b) {
@@ -215,7 +222,7 @@ __device__ __forceinline__ void store_block(const Acc (&acc)[MI][4], float *stag
                 o[r][h] = pack_bf2(bf2f(old[b][r][h] & 0xffff) + bf2f(o[r][h] & 0xffff),
                                    bf2f(old[b][r][h] >> 16) + bf2f(o[r][h] >> 16));
             }
-            stream_store<u32x4_a2_t>(o[r], row);
+            stream_store(o[r], row);
           } else {
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -242,7 +249,7 @@ __device__ __forceinline__ void store_block(const Acc (&acc)[MI][4], float *stag
           if constexpr (OUT == kOutI32) {
             int32_t *cp = static_cast<int32_t *>(C) + off;
             if (n + 4 <= N) {
-              stream_store<u32x4_a4_t>(__builtin_bit_cast(u32x4_t, acc[i][2 * jp + h]), cp);
+              stream_store(__builtin_bit_cast(u32x4_t, acc[i][2 * jp + h]), cp);
             } else {
 #pragma unroll
               for (int k = 0; k < 4; ++k) {
@@ -254,8 +261,8 @@ __device__ __forceinline__ void store_block(const Acc (&acc)[MI][4], float *stag
             float *cp = static_cast<float *>(C) + off;
             if (n + 4 <= N) {
               f32x4_t o = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
-              if constexpr (ACCUM) o += stream_load<f32x4_a4_t>(cp);
-              stream_store<f32x4_a4_t>(o, cp);
+              if constexpr (ACCUM) o += stream_load(cp);
+              stream_store(o, cp);
             } else {
 #pragma unroll
               for (int k = 0; k < 4; ++k)
