@@ -60,6 +60,8 @@ int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, void *C,
 }  // namespace
 }  // namespace vdnh3
 
+extern "C" int vdnh3_gemm_tile_rows(int M, int N) { return M > 0 && N > 0 ? 32 * vdnh3::gemm_mi(M, N) : 0; }
+
 extern "C" int vdnh3_gemm(int kind, const void *A, int64_t lda, const void *B, int64_t ldb, void *C, int64_t ldc,
                           int M, int N, int K, const float *a_scale, int a_scale_n, const float *b_scale,
                           int b_scale_n, float alpha, const void *bias, int bias_bf16, int act, int out_type,

@@ -63,6 +63,7 @@ SIGNATURES = {
                                           _c_size, _vp]),
     "vdnh3_gemm": (_c_int, [_c_int, _vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_int, _c_int, _c_int,
                             _vp, _c_int, _vp, _c_int, _c_float, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
+    "vdnh3_gemm_tile_rows": (_c_int, [_c_int, _c_int]),
     "vdnh3_quant_rows": (_c_int, [_c_int, _vp, _c_i64, _c_int, _c_int, _vp, _c_i64, _vp, _vp]),
     "vdnh3_quant_tensor_f8": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp]),
     "vdnh3_quant_tensor_f8_noalloc": (_c_int, [_vp, _c_i64, _vp, _vp, _vp]),

@@ -202,6 +202,9 @@ int vdnh3_gemm(int kind, const void *A, int64_t lda, const void *B, int64_t ldb,
                int b_scale_n, float alpha, const void *bias, int bias_bf16, int act, int out_type,
                int accumulate, int round_linear, void *stream);
 
+/* The rows of the output tiles vdnh3_gemm takes for an M x N output (its results don't depend on them). */
+int vdnh3_gemm_tile_rows(int M, int N);
+
 /*
  * Row-wise symmetric quantisation of a bf16 [M, K] matrix: kind 1 = int8 (scale amax/127,
  * round half to even, clamp +-127), kind 2 = fp8 e4m3fn (scale amax/448, clamp +-448,

@@ -240,11 +240,22 @@ def test_full_shape_int8_out_projection_sampled(device):
     assert_bf16_close(out[rows.to(device)], want, steps=1)
 
 
-# one size per tile height the launcher can pick (32 mi rows: the fewest rounds over 256 CUs), each with a ragged
-# last tile row, N a multiple of 8, of 4 and odd (the three store widths), and 1 to 5 stages of 128 K bytes
+# sizes of every tile height the launcher can pick (32 mi rows: the fewest rounds over 256 CUs), each with a ragged
+# last tile row, N a multiple of 8, of 4 and odd (whole and partly stored last columns), and 1 to 5 stages of 128 K
+# bytes
+TILE_SIZES = [(1, 8), (31, 20), (65, 257), (511, 15100), (1000, 5113), (513, 15100), (1801, 5113), (2303, 5116),
+              (2561, 5120), (2881, 4900), (4100, 5128)]
+
+
+def test_tile_sizes_cover_every_height():
+    from vdn_h3_amd import _lib
+
+    heights = {_lib.lib().vdnh3_gemm_tile_rows(m, n) for m, n in TILE_SIZES}
+    assert heights == {32 * mi for mi in (2, 4, 5, 6, 7, 8)}
+
+
 @pytest.mark.parametrize("stages", [1, 2, 3, 5])
-@pytest.mark.parametrize("m,n", [(1, 8), (31, 20), (65, 257), (513, 15100), (1801, 5113), (2303, 5116), (2561, 5120),
-                                 (2881, 4900), (4100, 5128)])
+@pytest.mark.parametrize("m,n", TILE_SIZES)
 def test_tile_heights_widths_and_stages(device, m, n, stages):
     from vdn_h3_amd import linear
 
