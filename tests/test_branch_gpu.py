@@ -154,8 +154,9 @@ def test_scans(device, text):
     _close(s, ws, 1e-4, 1e-5, "suffix")
 
 
-# one step, odd and even step counts, and item counts (heads x 2 x dim / 32) below, off and at a multiple of 8
-@pytest.mark.parametrize("frames,heads,dim", [(1, 1, 64), (2, 3, 128), (5, 2, 64), (6, 5, 128)])
+# one step, odd and even step counts, and item counts (heads x 2 x dim / 32) below 8, at a multiple of 8 and off one with
+# more than one item per XCD (12 and 52: workgroups left over)
+@pytest.mark.parametrize("frames,heads,dim", [(1, 1, 64), (2, 3, 128), (5, 2, 64), (6, 5, 128), (5, 3, 64), (4, 13, 64)])
 def test_scan_steps_and_item_counts(device, frames, heads, dim):
     from vdn_h3_amd import branch
 
