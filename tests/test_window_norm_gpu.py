@@ -119,6 +119,40 @@ def test_fused_attention_matches_separate(device, dim, rot, shared, gated):
     assert torch.equal(got.cpu().view(torch.int16), want.cpu().view(torch.int16))
 
 
+@pytest.mark.parametrize("dim,rot,shared", [(128, None, False), (64, None, False), (128, 64, False), (64, 64, True)])
+@pytest.mark.parametrize("block_m,splits", [(256, 3), (64, 4)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_fused_attention_with_split_keys(device, dim, rot, shared, block_m, splits, gated):
+    """The norm fused in and a plan with key splits: the bits of the separate pass on the same plan, at the oracle's bar."""
+    from vdn_h3_amd import window
+    from vdn_h3_amd.hybrid import normalise_qk
+
+    geo = _geometry(frames=9, per_frame=61, text=37)
+    seq, heads = geo["seq"], 3
+    q_eps, k_eps = 1e-6, 1e-5 if rot is None else 1e-6
+    print(f"case fused attention split D={dim} rot={rot} block_m={block_m} splits={splits} gated={gated}", flush=True)
+    q, k, v, wq, wk = _inputs(seq, heads, dim, 700 + dim + (rot or 0), device)
+    freqs = None if rot is None else _freqs(1 if shared else seq, rot, 11).to(device)
+    gate = torch.sigmoid(torch.randn(seq, heads, generator=torch.Generator().manual_seed(6))).to(
+        torch.bfloat16).to(device) if gated else None
+    geometry = (geo["vs"], geo["ve"], geo["frames"], geo["per_frame"], geo["bounds"])
+    items, tiles, pairs = window.build_plan_host(seq, *geometry, "both", block_m)
+    assert splits <= int(items[:, 3].min())
+    plan = window.WindowPlan(items.to(device), tiles.to(device), items.shape[0], tiles.shape[0], pairs, block_m, splits)
+    qn, kn = normalise_qk(q, k, wq, wk, q_eps, rope_freqs=freqs, k_eps=k_eps)
+    args = (*geometry, dim ** -0.5, "both")
+    want = window.window_softmax_hip(qn, kn, v, *args, gate=gate, plan=plan)
+    got = window.window_softmax_normed(q, k, v, wq, wk, q_eps, k_eps, *args, rope_freqs=freqs, gate=gate, plan=plan)
+    assert torch.equal(got.cpu().view(torch.int16), want.cpu().view(torch.int16))
+    exact = wo.window_attention_grouped(qn.cpu(), kn.cpu(), v.cpu(), *args).float()
+    if gated:
+        exact = exact * gate.cpu().float()[..., None]
+    # probabilities rounded to bf16 (2^-9 each) weigh the values and their own sum: 2^-8 of the largest value; then the
+    # roundings of the output and of the gate's product
+    bound = 2.0 ** -8 * v.float().abs().max().item() + 2.0 ** -7 * exact.abs()
+    assert bool(((got.float().cpu() - exact).abs() <= bound).all())
+
+
 def test_fused_attention_full_shape(device):
     """The full window workload (40688 rows, 40 heads, 128 dims, RoPE on every row): the fused
     path gives the same bits as the separate q/k pass and attention."""
