@@ -293,3 +293,32 @@ def test_tile_heights_widths_and_stages(device, m, n, stages):
         bound = (2.0 ** -14 if kind == "fp8" else k * 2.0 ** -24) * (ad.abs() @ bd.abs().t())
         assert bool(((got.double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()), kind
         assert torch.equal(out, (base.float() + got.float()).to(torch.bfloat16)), kind
+
+
+@pytest.mark.parametrize("m,n", TILE_SIZES)
+def test_32_bit_outputs_any_alignment(device, m, n):
+    """fp32 and int32 outputs, written and accumulated, into rows of any 4-byte alignment; the rest of them untouched."""
+    from vdn_h3_amd import linear
+
+    print(f"case 32-bit outputs {m}x{n}", flush=True)
+    k = 256
+    g = torch.Generator(device="cuda").manual_seed(m + 3 * n)
+    a = torch.randint(-127, 128, (m, k), generator=g, device=device, dtype=torch.int8)
+    b = torch.randint(-127, 128, (n, k), generator=g, device=device, dtype=torch.int8)
+    a_s = torch.rand(m, 1, generator=g, device=device) * 1e-2
+    b_s = torch.rand(1, n, generator=g, device=device) * 1e-2
+    acc = a.float() @ b.float().t()  # at most 256 products below 2^14: exact in fp32
+    base = torch.randn(m, n + 3, generator=g, device=device)
+    for first in (0, 1, 2, 3):
+        for accumulate in (False, True):
+            whole = base.clone()
+            out = whole[:, first:first + n]
+            linear.gemm_w8a8(a, a_s, b, b_s, out=out, out_dtype=torch.float32, accumulate=accumulate)
+            want = base.clone()
+            want[:, first:first + n] = acc * a_s * b_s + (base[:, first:first + n] if accumulate else 0)
+            assert torch.equal(whole, want), (first, accumulate)
+        ints = torch.full((m, n + 3), 7, dtype=torch.int32, device=device)
+        linear.gemm(linear.KIND_I8, a, b, out=ints[:, first:first + n], out_dtype=torch.int32)
+        want = torch.full_like(ints, 7)
+        want[:, first:first + n] = acc.to(torch.int32)
+        assert torch.equal(ints, want), first
