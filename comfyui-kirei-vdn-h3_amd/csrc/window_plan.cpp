@@ -10,6 +10,7 @@
 // and last tile of an interval carry a column mask.
 #include <algorithm>
 #include <cstdint>
+#include <functional>
 #include <vector>
 
 #include "common.h"
@@ -144,47 +145,76 @@ Plan make_plan(const Geometry &g, int block_m, int block_n) {
 
 // How a call with `heads` heads is best divided: the most query rows of an item (256, 128 or 64) and how many
 // workgroups share an item's key tiles, by the least estimated time. A workgroup takes its tiles plus about five
-// (prologue, first loads, epilogue), one workgroup per CU; more than 256 of them share the CUs evenly with
-// half the longest left over. us per tile and workgroup, measured at 4, 9 and 70 tiles: 1.95 / 1.68 / 1.62 with 256
-// / 128 / 64 rows at head dim 128, 1.50 / 1.23 / 1.17 at 64 (below 129 rows one of the workgroup's two groups is
-// idle and the other's phases have the SIMDs to themselves). Splits cost a combining launch (12 us with its host
-// side) and their fp32 partials written and read (about 6 TB/s). Whole items of 256 rows stay unless 5% are gained,
-// so a call that fills the GPU is left as it is. Measured, whole items of 256 rows against the choice: one head of
-// 6,700 rows 151 -> 43 us (8 splits), one head of 40,688 rows 850 -> 630 us, four heads of 6,700 rows 158 -> 98 us,
-// two heads of 848 rows of 64 (64 rows an item, whole) 21 -> 16 us.
+// (prologue, first loads, epilogue), one workgroup per CU. An XCD's 32 CUs run the splits of its own eighth of the
+// items, as the kernel numbers them (head by head, longest first, all first splits before the second ones), and nobody
+// else's; the estimate gives each in turn to the CU that is free first and takes the slowest XCD. us per tile and
+// workgroup, measured at 4, 9 and 70 tiles: 1.95 / 1.68 / 1.62 with 256 / 128 / 64 rows at head dim 128, 1.50 / 1.23 /
+// 1.17 at 64 (below 129 rows one of the workgroup's two groups is idle and the other's phases have the SIMDs to
+// themselves). Splits cost a combining launch (9 us with its host side) and their fp32 partials written and read (about
+// 6 TB/s). Whole items of 256 rows stay unless 5% are gained; calls of 1,024 items or more fill the GPU and are left as
+// they are. Over 500 timings of drawn calls the estimate is within 7% (2-norm); with the work spread evenly over all
+// 256 CUs it was within 20% for split calls, and one call in sixty took 3 to 10% longer than whole items. Whole items
+// of 256 rows against the choice: one head of 6,700 rows 151 -> 44 us, four heads of 6,700 rows 158 -> 98 us, two heads of
+// 848 rows of 64 (64 rows an item, whole) 21 -> 16 us.
 struct Shape {
   int block_m, splits;
 };
+
+constexpr int kXcds = 8, kXcdCus = 32;
+constexpr int kMostWorkgroups = 2048;  // splits beyond eight rounds of the CUs even nothing out
+
+// The tiles' worth of time an XCD takes for `s` splits of these items, or any time >= `limit` it takes at least.
+int64_t xcd_tiles(const int64_t *items, int64_t n, int s, int64_t limit) {
+  auto length = [&](int64_t tiles, int y) { return tiles * (y + 1) / s - tiles * y / s + 5; };
+  int64_t longest = 0, work = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    longest = std::max(longest, (items[i] + s - 1) / s + 5);
+    work += items[i] + 5 * s;
+  }
+  const int64_t least = std::max(longest, (work + kXcdCus - 1) / kXcdCus);
+  if (n * s <= kXcdCus || least >= limit) return least;
+  int64_t free_at[kXcdCus] = {}, end = 0;  // a heap, the CU that is free first in front
+  for (int y = 0; y < s; ++y)
+    for (int64_t i = 0; i < n; ++i) {
+      std::pop_heap(free_at, free_at + kXcdCus, std::greater<int64_t>());
+      int64_t &t = free_at[kXcdCus - 1];
+      t += length(items[i], y);
+      end = std::max(end, t);
+      std::push_heap(free_at, free_at + kXcdCus, std::greater<int64_t>());
+    }
+  return end;
+}
 
 Shape shape_call(const std::vector<Run> &runs, int block_n, int64_t heads, int seq, int dim) {
   struct Count {
     int64_t rows, tiles;
   };
   std::vector<Count> counts;
-  int64_t fewest = INT64_MAX, most = 0;
+  int64_t fewest = INT64_MAX, items_256 = 0;
   for (const Run &r : runs) {
     std::vector<int32_t> tiles;
     tiles_of(r.keys, block_n, &tiles);
-    const int64_t n = int64_t(tiles.size() / 2);
-    counts.push_back({r.q1 - r.q0, n});
-    fewest = std::min(fewest, n);
-    most = std::max(most, n);
+    counts.push_back({r.q1 - r.q0, int64_t(tiles.size() / 2)});
+    fewest = std::min(fewest, counts.back().tiles);
+    items_256 += (r.q1 - r.q0 + 255) / 256;
   }
   Shape best{256, 1};
+  if (items_256 * heads >= 1024) return best;
+  std::stable_sort(counts.begin(), counts.end(), [](const Count &x, const Count &y) { return x.tiles > y.tiles; });
   double best_us = -1;
   for (const int bm : {256, 128, 64}) {
-    int64_t items = 0, work = 0;
-    for (const Count &c : counts) {
-      const int64_t n = (c.rows + bm - 1) / bm;
-      items += n;
-      work += n * c.tiles;
-    }
+    std::vector<int64_t> items;  // the tiles of every head's items, longest first per head
+    for (int64_t h = 0; h < heads; ++h)
+      for (const Count &c : counts) items.insert(items.end(), (c.rows + bm - 1) / bm, c.tiles);
+    const int64_t total = items.size(), per_xcd = (total + kXcds - 1) / kXcds;
     const double tile_us = dim > 64 ? (bm == 256 ? 1.95 : bm == 128 ? 1.68 : 1.62) : (bm == 256 ? 1.50 : bm == 128 ? 1.23 : 1.17);
-    for (int s = 1; s <= std::min<int64_t>(fewest, 16); ++s) {
-      const double longest = double(most) / s + 5;
-      double us = items * heads * s <= 256 ? longest : double(work + 5 * s * items) * heads / 256 + longest / 2;
-      us *= tile_us;
-      if (s > 1) us += 12 + 8e-6 * s * heads * seq * dim / 6;
+    for (int s = 1; s <= std::min<int64_t>(fewest, 16) && (s == 1 || total * s <= kMostWorkgroups); ++s) {
+      const double combine_us = s > 1 ? 9 + 8e-6 * s * heads * seq * dim / 6 : 0;
+      const int64_t limit = best_us < 0 ? INT64_MAX : int64_t((best_us - combine_us) / tile_us) + 1;
+      int64_t tiles = 0;
+      for (int64_t first = 0; first < total && tiles < limit; first += per_xcd)
+        tiles = std::max(tiles, xcd_tiles(&items[first], std::min(per_xcd, total - first), s, limit));
+      const double us = tiles * tile_us + combine_us;
       if (best_us < 0) best_us = 0.95 * us;  // whole items of 256 rows
       else if (us < best_us) best = {bm, s}, best_us = us;
     }

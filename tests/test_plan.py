@@ -103,3 +103,19 @@ def test_cached_plan_whatever_holds_the_bounds(built_lib, hold):
     for wrong in ([(0, 1, 2), (3,)], [(0,)] * 5, []):
         with pytest.raises(ValueError):
             cache.plan(*geometry(wrong))
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("seq,heads", [(6700, 1), (8364, 1), (10598, 2), (16441, 3), (23883, 2), (23883, 5), (40688, 1),
+                                       (40688, 3), (40688, 5)])
+def test_key_splits_save_rounds(built_lib, seq, heads, dim):
+    """Items of one length: an XCD's 32 CUs take its eighth of the items' splits in rounds, and a choice with splits takes
+    less in those rounds than whole items do (33 workgroups on an XCD are two rounds)."""
+    from vdn_h3_amd import window
+
+    def rounds(block_m, splits):
+        per_xcd = -(-(-(-seq // block_m) * heads) // 8)
+        return -(-per_xcd * splits // 32) * (-(-seq // 96) / splits + 5)
+
+    plan = window.make_plan(seq, 0, seq, 1, seq, [(0, 0)], "none", torch.device("cpu"), heads, dim)
+    assert (plan.block_m, plan.splits) == (256, 1) or rounds(plan.block_m, plan.splits) < rounds(256, 1)
