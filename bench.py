@@ -580,12 +580,13 @@ CPU_THREADS = 16   # host threads of the CPU baseline: the host's CPU share for 
 
 
 MFMA_KINDS = {0: ("bf16_32x32x16", PEAK_BF16_TFLOPS), 1: ("int8_32x32x32", PEAK_I8_TOPS),
-              2: ("fp8_e4m3_32x32x64", PEAK_F8_TFLOPS)}
+              2: ("fp8_e4m3_32x32x64", PEAK_F8_TFLOPS), 3: ("bf16_16x16x32", PEAK_BF16_TFLOPS),
+              4: ("int8_16x16x64", PEAK_I8_TOPS), 5: ("fp8_e4m3_16x16x128", PEAK_F8_TFLOPS)}
 
 
 def mfma_rate(torch, device, kind, data="random", reps=3, warmup=1):
     """Sustained MFMA rate (T(FL)OP/s, median of ``reps`` launches of 10-20 ms) of ``kind`` (0 bf16,
-    1 int8, 2 fp8 e4m3) on register-resident operands (vdnh3_mfma_peak): random operands (what the
+    1 int8, 2 fp8 e4m3 in their 32x32 shapes, 3 to 5 in their 16x16 ones) on register-resident operands (vdnh3_mfma_peak): random operands (what the
     kernels see: bf16 N(0,1), int8 uniform in [-127, 127], e4m3 codes of N(0,1)) or zeros, two
     workgroups of 4 wavefronts per CU, independent accumulators."""
     from vdn_h3_amd import _lib
@@ -597,16 +598,16 @@ def mfma_rate(torch, device, kind, data="random", reps=3, warmup=1):
     gen = torch.Generator().manual_seed(20261202)
     if data == "zero":
         src = torch.zeros(n, dtype=torch.uint8)
-    elif kind == 0:
+    elif kind % 3 == 0:
         src = torch.randn(n // 2, generator=gen).to(torch.bfloat16).view(torch.uint8)
-    elif kind == 1:
+    elif kind % 3 == 1:
         src = torch.randint(-127, 128, (n,), generator=gen, dtype=torch.int8).view(torch.uint8)
     else:
         src = torch.randn(n, generator=gen).to(torch.float8_e4m3fn).view(torch.uint8)
     cus = torch.cuda.get_device_properties(device).multi_processor_count
     blocks = 2 * cus  # one round: two workgroups per CU for the whole run
     out = torch.empty(blocks * 256, dtype=torch.float32, device=device)
-    iters = {0: 40000, 1: 40000, 2: 20000}[kind]
+    iters = {0: 40000, 1: 40000, 2: 20000}.get(kind, 10000)
     ops = lib.vdnh3_mfma_peak_ops(kind, iters, blocks)
     a, b = src.to(device), src.roll(4096).to(device)
 
@@ -629,11 +630,11 @@ def mfma_rate(torch, device, kind, data="random", reps=3, warmup=1):
 
 
 def ceiling_entry(torch, device, kind, achieved):
-    """The kernel's rate against the part's sustained random-operand MFMA rate of the same kind,
-    measured after the timed region (the datasheet ``roofline.peak`` assumes a clock the part holds
+    """The kernel's rate against the part's sustained random-operand MFMA rate of the same kind, in the 16x16
+    shape the kernels use, measured after the timed region (the datasheet ``roofline.peak`` assumes a clock the part holds
     only on operands that barely toggle)."""
-    rate, _ = mfma_rate(torch, device, kind)
-    return {"mfma": MFMA_KINDS[kind][0], "operands": "random", "rate": round(rate, 1),
+    rate, _ = mfma_rate(torch, device, kind + 3)
+    return {"mfma": MFMA_KINDS[kind + 3][0], "operands": "random", "rate": round(rate, 1),
             "achieved": round(achieved, 2), "frac": round(achieved / rate, 4),
             "source": "vdnh3_mfma_peak (bench.py --workload mfma_peak)"}
 
@@ -654,7 +655,7 @@ def bench_mfma_peak(args, torch, device):
         "unit": "TFLOP/s",
         "ms_per_step": rates["bf16_32x32x16_random"]["ms"],
         "dtype": "bf16/int8/fp8",
-        "config": {"workload": "mfma_peak", "blocks": 2 * cus, "waves_per_cu": 8, "mfmas_per_wave_iter": 8},
+        "config": {"workload": "mfma_peak", "blocks": 2 * cus, "waves_per_cu": 8, "mfmas_per_wave_iter": "8; 16x16 shapes 64, fp8 32"},
         "rates": rates,
     }
 

@@ -515,8 +515,9 @@ int vdnh3_fill_rows_bf16(uint16_t *p, int64_t ld, int rows, int cols, float valu
  * ------------------------------------------------------------------------------ */
 
 /* Runs `blocks` workgroups of 4 wavefronts, each issuing iters x 8 independent MFMAs of `kind`
- * (0 bf16 32x32x16, 1 int8 32x32x32, 2 fp8 e4m3 32x32x64) on register-resident fragments:
- * a and b hold 8 x 64 lanes x 32 bytes each (32-byte aligned; bf16 and int8 use the first 16
+ * (0 bf16 32x32x16, 1 int8 32x32x32, 2 fp8 e4m3 32x32x64) or iters x 64 (fp8 x 32) of the 16x16 shapes the GEMM
+ * and the attention use (3 bf16 16x16x32, 4 int8 16x16x64, 5 fp8 e4m3 16x16x128) on register-resident fragments:
+ * a and b hold 8 x 64 lanes x 32 bytes each (32-byte aligned; bf16 and int8 in the 32x32 shapes use the first 16
  * bytes of each lane's 32). out receives blocks x 256 floats (a checksum that keeps the work live). */
 int vdnh3_mfma_peak(int kind, const void *a, const void *b, int iters, int blocks, float *out, void *stream);
 

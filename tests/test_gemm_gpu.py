@@ -322,3 +322,21 @@ def test_32_bit_outputs_any_alignment(device, m, n):
         want = torch.full_like(ints, 7)
         want[:, first:first + n] = acc.to(torch.int32)
         assert torch.equal(ints, want), first
+
+
+@pytest.mark.parametrize("kind,dtype,k,per_lane", [
+    (0, torch.bfloat16, 16, 2), (1, torch.int8, 32, 2), (2, torch.float8_e4m3fn, 64, 2),        # 4 accumulators of 16
+    (3, torch.bfloat16, 32, 2), (4, torch.int8, 64, 2), (5, torch.float8_e4m3fn, 128, 1)])     # 32 accumulators of 4
+def test_mfma_rate_kernels_do_their_products(device, kind, dtype, k, per_lane):
+    """Operands of ones: a lane's checksum counts the products of its MFMAs (``per_lane`` on each accumulator a pass)."""
+    from vdn_h3_amd import _lib
+
+    iters, blocks = 3, 4
+    ones = torch.ones(8 * 64 * 32 // dtype.itemsize, dtype=torch.float32).to(dtype).to(device)
+    out = torch.empty(blocks * 256, dtype=torch.float32, device=device)
+    lib = _lib.lib()
+    _lib.check(lib.vdnh3_mfma_peak(kind, _lib.ptr(ones), _lib.ptr(ones), iters, blocks, _lib.ptr(out),
+                                   _lib.stream_handle(device)), "mfma_peak")
+    values = 4 * 16 if kind < 3 else 32 * 4
+    assert bool((out == values * per_lane * iters * k).all())
+    assert lib.vdnh3_mfma_peak_ops(kind, iters, blocks) == 2 * values * 64 * per_lane * iters * k * 4 * blocks
