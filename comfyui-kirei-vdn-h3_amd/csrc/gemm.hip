@@ -12,9 +12,12 @@ namespace vdnh3 {
 namespace {
 
 // Tile height (32 mi rows) for an M x N output: the one whose rounds of tiles over the 256 CUs, one workgroup
-// each, take least. A round costs about mi + 1.5: at 8192^3 in bf16 197 / 166 / 147 / 130 / 113 / 82 us for
-// mi = 8 / 7 / 6 / 5 / 4 / 2 (the B tile's loads and reads, the prologue and the epilogue do not shrink with
-// mi). Large outputs so keep mi = 8; in between the height follows the last round (8,296 x 5,120: mi = 7, three
+// each, take least. A round is taken to cost mi + 1.5 (the B tile's loads and reads, the prologue and the epilogue do
+// not shrink with mi). Measured, one round for mi = 8 / 7 / 6 / 5 / 4 / 2: 185 / 170 / 151 / 130 / 114 / 74 us with
+// 16,384 bytes of K in bf16, and for each type mi + 2 fits from 2,048 bytes on, mi + 3 512 bytes and mi + 4 one stage
+// of 128 (bf16 10.0 / 8.9 / 7.8 / 6.8 / 6.5 / 4.9 us). Over 20,000 sizes drawn up to 40,688 x 15,360 the choice by
+// mi + 2 differs for 0.6%, by at most 0.4% of the time, by mi + 4 for 1.1%, by at most 7%, so one line serves every
+// type and K. Large outputs keep mi = 8; in between the height follows the last round (8,296 x 5,120: mi = 7, three
 // full rounds, 346 us, against 348 with 8 and 2.6 rounds' worth of tiles; 1,808 x 5,120: mi = 5 79 us against 94;
 // 40,688 x 208: mi = 5 123 us against 141), and few rows take low tiles, which leave fewer CUs idle (512 x
 // 15,360 in int8: mi = 4 38.5 us against 50; 8,296 x 208: mi = 2 48 us against 101).

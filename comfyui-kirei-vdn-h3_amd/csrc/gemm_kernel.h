@@ -5,8 +5,8 @@
 //
 // Matrix instructions: the 16x16 shapes (v_mfma_f32_16x16x32_bf16, v_mfma_i32_16x16x64_i8,
 // v_mfma_f32_16x16x128_f8f6f4 without block scales). The part is limited by power, not by issue: on
-// random operands held in registers the 32x32 shapes run at 1740 / 3290 / 3890 T(FL)OP/s (bf16 / int8 / fp8)
-// and the 16x16 shapes, walked so that successive MFMAs share one operand, at 2003 / 3971 / 4288. With the
+// random operands held in registers (calib.hip) the 32x32 shapes run at 1750 / 3364 / 3903 T(FL)OP/s (bf16 / int8 /
+// fp8) and the 16x16 shapes, walked so that successive MFMAs share one operand, at 2003 / 3975 / 4214. With the
 // 32x32 shapes this GEMM's bf16 8192^3 kept the MFMA pipes busy 0.78 of the cycles at 1.48 GHz.
 //
 // Tiling: a workgroup of 8 wavefronts (two per SIMD, so that one wavefront's MFMAs issue while the other
@@ -333,11 +333,11 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_nt_kernel(const GemmArgs
   constexpr int A_STAGE = BM * kGemmSK, B_STAGE = kGemmBN * kGemmSK;
   constexpr int A_WL = BM / 8;  // an A stage in wavefront loads (8 rows, 1 KB each)
   constexpr int NA = (A_WL + 7) / 8, NB = kGemmBN / 64, NL = NA + NB;  // loads per wavefront and stage
-  // loads per unit from the barrier on; all go out at least half a stage before the barrier that waits for them
   // Stages s + 1 .. s + D are in flight or landed while stage s is multiplied, through D + 2 slots for A and D + 1
   // for B: 160 KB for MI = 8, D = 1. A tile of at most 128 rows has its stage's MFMAs done before a load issued
   // one stage ahead returns, and LDS to spare.
   constexpr int D = MI <= 4 ? 2 : 1, SA = D + 2, SB = D + 1;
+  // loads per unit from the barrier on; all go out at least half a stage before the barrier that waits for them
   constexpr int LPU = U == 2 ? 3 : KIND == kF8 || U < 2 * NL ? 2 : 1;
   static_assert(U % R == 0 && RA <= R && U * LPU >= NL, "fragment ring and load slots");
   __shared__ __attribute__((aligned(16))) uint8_t smem[SA * A_STAGE + SB * B_STAGE];

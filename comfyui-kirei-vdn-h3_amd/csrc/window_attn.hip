@@ -11,7 +11,7 @@
 //   then owns one query of each 16-query block (lane % 16) and 24 of the 96 keys of a tile, so the row
 //   maxima take three lane swaps and the probabilities P^T feed the next MFMA (O^T += V^T P^T)
 //   straight from registers, without an LDS round trip. The 16x16 shape does the same work at 13% less
-//   power than 32x32x16 (register-only rates 2003 against 1740 TFLOP/s on random operands), and this kernel
+//   power than 32x32x16 (register-only rates 2003 against 1750 TFLOP/s on random operands), and this kernel
 //   is power-bound: with the row sums below, 15.55 -> 15.02 ms at 40,688 x 40 x 128 and 2510 -> 2368 us at
 //   16,007 x 56 x 128 (72 frames of 209 tokens), alternated on one machine.
 //   V^T is read from a copy made by a pre-pass (one extra 2*S*H*D-byte sweep): per head, one
@@ -35,7 +35,7 @@ namespace vdnh3 {
 namespace {
 
 constexpr int kBM = 256;  // query rows per workgroup (8 wavefronts x 32)
-constexpr int kBN = 96;   // keys per tile: 48 MFMAs per wavefront and phase at D = 128
+constexpr int kBN = 96;   // keys per tile: 102 MFMAs per wavefront and phase at D = 128
 constexpr int kThreads = 512;
 constexpr int kRing = 3;  // LDS slots per K and V^T ring (144 KB at D = 128): loads run kRing - 1 tiles ahead
 // fragments a wavefront's LDS reads run ahead of its MFMAs: 8 / 6 / 5 / 4 measured 15.45 / 15.31 / 15.17 / 15.39 ms

@@ -290,6 +290,10 @@ def window_softmax_hip(query, key, value, video_start, video_end, num_frames, to
     Head dims other than 64 and 128 (up to 128; the reference's op is shape-generic,
     ``vdn_h3/window.py:277-313``) run at the next kernel head dim with zero channels added to q, k and v:
     a zero channel adds nothing to a score and yields a zero output channel, and ``scale`` is the caller's.
+    Calls of few heads divide the keys of a row over workgroups (``make_plan``): they take fp32 partial results
+    (``splits * H * S * (D + 2)`` values) while they run, and a head's last bits then depend on how many heads
+    are computed with it. ``plan=make_plan(...)`` made without ``heads`` keeps the rows whole: a head's bits are then
+    the same in any company.
     """
     _check_qkv(query, key, value, "window_softmax_hip")
     _lib.forward_only("window_softmax_hip", query, key, value, gate)

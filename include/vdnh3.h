@@ -69,7 +69,8 @@ int vdnh3_window_plan_build(int seq, int video_start, int video_end, int num_fra
                             int block_m, int block_n, int32_t *items, int32_t n_items,
                             int32_t *tiles, int32_t n_tiles);
 
-/* The item height (block_m: 256, 128 or 64 rows) and the number of key splits that suit a call with `heads` heads. */
+/* The item height (block_m: 256, 128 or 64 rows; no effect on the result) and the number of key splits that suit a call
+ * with `heads` heads. */
 int vdnh3_window_plan_shape(int seq, int video_start, int video_end, int num_frames, int tokens_per_frame,
                             const int32_t *bounds, int anchor_mode, int block_n, int heads, int head_dim,
                             int32_t *block_m, int32_t *splits);
@@ -123,7 +124,8 @@ int vdnh3_window_attn_prepared(const uint16_t *q, int64_t q_row, int64_t q_head,
 /*
  * The same with each work item's key tiles divided over `splits` workgroups (1 to 64; those past an item's tile
  * count add nothing), whose partial results are combined by a second kernel: for calls with too few work
- * items to fill the GPU. `partial` holds vdnh3_window_partial_bytes (unused with splits = 1).
+ * items to fill the GPU. `partial` holds vdnh3_window_partial_bytes (unused with splits = 1). Each split rounds its
+ * probabilities against its own running max, so the number of splits shows in the last bits of the result.
  */
 size_t vdnh3_window_partial_bytes(int seq, int heads, int head_dim, int splits);
 int vdnh3_window_attn_prepared_split(const uint16_t *q, int64_t q_row, int64_t q_head,
@@ -133,7 +135,7 @@ int vdnh3_window_attn_prepared_split(const uint16_t *q, int64_t q_row, int64_t q
                                int seq, int heads, int head_dim, float scale,
                                const int32_t *items, int32_t n_items, const int32_t *tiles,
                                const void *workspace, size_t workspace_bytes, int splits,
-    float *partial, size_t partial_bytes, void *stream);
+                               float *partial, size_t partial_bytes, void *stream);
 
 /*
  * The attention with the block's q_norm / k_norm fused in (vdn_h3/hybrid.py:271-292 followed by
@@ -170,7 +172,7 @@ int vdnh3_window_attn_qnorm_split(const uint16_t *q, int64_t q_row, int64_t q_he
                             uint16_t *out, int64_t o_row, int64_t o_head, const uint16_t *gate, int64_t gate_row,
                             int seq, int heads, int head_dim, float scale, const int32_t *items, int32_t n_items,
                             const int32_t *tiles, const void *workspace, size_t workspace_bytes, int splits,
-    float *partial, size_t partial_bytes, void *stream);
+                            float *partial, size_t partial_bytes, void *stream);
 
 /* ------------------------------------------------------------------------------
  * Projections (reference vdn_h3/projection.py, vdn_h3/fp8.py, the block's qkv/out GEMMs)

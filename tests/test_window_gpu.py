@@ -316,3 +316,21 @@ def test_items_stay_whole_without_memory_for_partials(device, monkeypatch, norme
     monkeypatch.setattr(torch, "empty", full)
     out = call(plan)
     assert refused and torch.equal(out, whole) and not torch.equal(split, whole)
+
+
+def test_whole_items_keep_a_heads_bits_in_any_company(device):
+    """With a plan made without the number of heads a head computed alone has the bits it has among others."""
+    from vdn_h3_amd import window
+
+    frames, per_frame, text, heads, dim = 13, 300, 100, 6, 128
+    seq = text + frames * per_frame
+    geometry = (text, seq, frames, per_frame, wo.window_bounds(frames, 1, 5))
+    gen = torch.Generator().manual_seed(37)
+    q, k, v = (torch.randn(seq, heads, dim, generator=gen).to(torch.bfloat16).to(device) for _ in range(3))
+    plan = window.make_plan(seq, *geometry, "both", device)
+    assert plan.splits == 1 and window.make_plan(seq, *geometry, "both", device, 1, dim).splits > 1
+    args = (*geometry, dim ** -0.5, "both")
+    together = window.window_softmax_hip(q, k, v, *args, plan=plan)
+    for head in (0, heads - 1):
+        alone = window.window_softmax_hip(*(t[:, head:head + 1] for t in (q, k, v)), *args, plan=plan)
+        assert torch.equal(alone, together[:, head:head + 1])
