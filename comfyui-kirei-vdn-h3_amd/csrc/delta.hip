@@ -232,7 +232,7 @@ __global__ __launch_bounds__(256, 2) void frame_stats_kernel(const StatsJob job,
 // The pivots are a chain of barriers and LDS round trips (about 1500 cycles each), so what counts is how many
 // matrices a CU works on at once: M is staged for J in halves of 64 columns, 34 KB of LDS instead of 67, and the
 // registers stay within 128, four workgroups per CU instead of two: 1,400 matrices of 128 x 128 in 210 us instead
-// of 260. A launch takes up to two jobs (the video frames and the text state, whose 40 matrices alone cost a
+// of 260 (up to 512, one round of two a CU, take 69 instead of 67). A launch takes up to two jobs (the video frames and the text state, whose 40 matrices alone cost a
 // whole chain, 68 us).
 struct FactorJob {
   const float *A, *B, *alpha;

@@ -13,7 +13,8 @@
 //   straight from registers, without an LDS round trip. The 16x16 shape does the same work at 13% less
 //   power than 32x32x16 (register-only rates 2003 against 1750 TFLOP/s on random operands), and this kernel
 //   is power-bound: with the row sums below, 15.55 -> 15.02 ms at 40,688 x 40 x 128 and 2510 -> 2368 us at
-//   16,007 x 56 x 128 (72 frames of 209 tokens), alternated on one machine.
+//   16,007 x 56 x 128 (72 frames of 209 tokens), alternated on one machine. Where at most one workgroup a CU runs the
+//   clock has room and the shape takes 2-4% longer (2,180 x 16 x 128 57.5 us against 55.9).
 //   V^T is read from a copy made by a pre-pass (one extra 2*S*H*D-byte sweep): per head, one
 //   contiguous image per 96-key tile, its 16-byte chunks already in the order and XOR swizzle of
 //   the kernel's LDS tile, with keys interleaved in 16-key groups so that each lane's 8 MFMA
