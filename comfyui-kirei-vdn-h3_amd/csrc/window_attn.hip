@@ -45,8 +45,8 @@ constexpr int kAhead = 4;
 constexpr float kLazy = 8.0f;  // log2 of the largest probability a stale running max allows
 // The running max before the first score above it. Finite, so that a tile whose scores are all -inf (keys masked
 // through a channel of q and k) adds zeros and not exp2(-inf + inf); and above every masked score of a type's
-// lowest value, whose rounded product with the scale is no maximum to subtract (its last place exceeds 2^128). A row
-// with no score above it has no sum: 0 / 0, NaN, as of a row of -inf.
+// lowest value, whose rounded product with the scale is no maximum to subtract: it is off by up to half its last place,
+// and exp2 overflows at 128. A row with no score above it has no sum: 0 / 0, NaN, as of a row of -inf.
 constexpr float kNoMax = -2147483648.0f;
 
 // LDS position p (0..31) of V^T inside a 32-key group holds key offset kperm(p): the order in which lane
